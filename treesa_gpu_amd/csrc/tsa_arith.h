@@ -246,10 +246,31 @@ TSA_HD float tsa_energy_from_counts(const TsaCounts& c, const TsaModel& P, const
   return w * (float)(sc1 - sc0) + dtc;
 }
 
+// Half-width of the band around the hardware's estimate of ln u in which tsa_metropolis evaluates expf.
+#define TSA_LN_BAND 2e-5f
+#if defined(__HIPCC__)
+// The hardware's estimate of ln u for u = (r >> 8) * 2^-24 (v_log_f32; -inf for u = 0).
+__device__ __forceinline__ float tsa_ln_estimate(uint32_t r) {
+  return __builtin_amdgcn_logf((float)(r >> 8) * (1.0f / 16777216.0f)) * 0.693147181f;
+}
+#endif
+
 // Metropolis: u = (r >> 8) * 2^-24 < expf(-beta * dE).  common.h:226-229.
+// On the device the decision is taken from an estimate t of ln u where it is certain: {x : expf(x) > u} is every
+// float from its least element T(u) up (expf is non-decreasing over the floats), and T(u) lies within
+// TSA_LN_BAND * (1 - t) of t for every u > 0 (checked for all of them on the device, bin/tsa_mathcheck).  Only an x
+// inside that band (about one visit in 10^4), a NaN and u = 0 take expf: a visit's exponential is some 30
+// instructions, half of them double, against 8 here.
 TSA_HD bool tsa_metropolis(uint32_t r, float beta, float dE, const uint64_t* exp2tab) {
   const float u = (float)(r >> 8) * (1.0f / 16777216.0f);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float x = -beta * dE, t = tsa_ln_estimate(r), band = TSA_LN_BAND * (1.0f - t);
+  bool acc = x > t + band;
+  if (!(acc || x < t - band)) acc = u < tsa_expf_t(x, exp2tab);
+  return acc;
+#else
   return u < tsa_expf_t(-beta * dE, exp2tab);
+#endif
 }
 
 // The Metropolis test as a threshold on x = -beta * dE: tsa_expf is non-decreasing over the floats (checked on

@@ -76,6 +76,15 @@ __global__ void __launch_bounds__(256) k_thr(uint32_t n, float* __restrict__ out
     out[k] = tsa_accept_threshold(k << 8, tab);
 }
 
+// out[k] = how far the threshold lies from the estimate of ln u that the Metropolis test decides by, as a share of
+// the band around it in which the test evaluates expf (0 for u = 0: the band is infinite)
+__global__ void __launch_bounds__(256) k_band(uint32_t n, const float* __restrict__ thr, float* __restrict__ out) {
+  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    const float t = tsa_ln_estimate(k << 8);
+    out[k] = k == 0 ? 0.0f : fabsf(thr[k] - t) / (TSA_LN_BAND * (1.0f - t));
+  }
+}
+
 static unsigned host_threads() {
   const unsigned n = std::thread::hardware_concurrency();
   return n == 0 ? 4 : (n > 16 ? 16 : n);
@@ -182,14 +191,24 @@ int main() {
     return (long long)(!same(h1[k], want) || h1[k] != h1[k]);
   });
 
+  // the test's band around the hardware's ln u: every threshold well inside it (a quarter, so that the rounding of
+  // the band's own ends cannot matter)
+  hipLaunchKernelGGL(k_band, grid, block, 0, 0, nthr, d1, d2);
+  CK(hipGetLastError());
+  CK(hipMemcpy(h2, d2, (size_t)nthr * 4, hipMemcpyDeviceToHost));
+  const long long bad_band = parallel_count(nthr, [&](uint32_t k) { return (long long)!(h2[k] <= 0.25f); });
+  float band_most = 0.0f;
+  for (uint32_t k = 0; k < nthr; k++) band_most = h2[k] > band_most ? h2[k] : band_most;
+
   printf("{\"expf_mismatch\": %lld, \"exp2f_mismatch\": %lld, \"exp_inputs\": %llu, \"log2f_mismatch\": %lld, "
          "\"log2f_inputs\": %u, \"lse_mismatch\": %lld, \"lse_inputs\": %lld, \"threshold_mismatch\": %lld, "
-         "\"threshold_inputs\": %u, \"host_threads\": %u}\n",
-         bad_exp, bad_exp2, 1ull << 32, bad_log2, nlog, bad_lse, n_lse, bad_thr, nthr, host_threads());
+         "\"threshold_inputs\": %u, \"band_mismatch\": %lld, \"band_most\": %g, \"host_threads\": %u}\n",
+         bad_exp, bad_exp2, 1ull << 32, bad_log2, nlog, bad_lse, n_lse, bad_thr, nthr, bad_band,
+         (double)band_most, host_threads());
   CK(hipFree(d1));
   CK(hipFree(d2));
   CK(hipFree(dfix));
   CK(hipHostFree(h1));
   CK(hipHostFree(h2));
-  return bad_exp || bad_exp2 || bad_log2 || bad_lse || bad_thr ? 1 : 0;
+  return bad_exp || bad_exp2 || bad_log2 || bad_lse || bad_thr || bad_band ? 1 : 0;
 }
