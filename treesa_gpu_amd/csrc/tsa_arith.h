@@ -97,19 +97,23 @@ TSA_HD float tsa_lse_i(int a, int b, const float* lse) {
 }
 
 // log2 of the modeled time of one contraction, GPU roofline model (common.h:129-135).
-TSA_HD float tsa_gpu_lt(int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
+// lab = lse_f of the two operands' sizes B+M+K and B+N+K (both models fold those first).
+TSA_HD float tsa_gpu_lt_from(float lab, int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
   const int Me = M > P.m0 ? M : P.m0, Ne = N > P.n0 ? N : P.n0, Ke = K > P.k0 ? K : P.k0;
   const float lops = (float)(1 + B + Me + Ne + Ke) - P.lpeak;
-  const float lbits = tsa_lse_f(tsa_lse_f((float)(B + M + K), (float)(B + N + K), T), (float)(B + M + N), T) - P.lbw;
+  const float lbits = tsa_lse_f(lab, (float)(B + M + N), T) - P.lbw;
   const float lt = lops > lbits ? lops : lbits;
   return tsa_lse_f(lt, P.llaunch, T);
 }
+TSA_HD float tsa_gpu_lt(int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
+  return tsa_gpu_lt_from(tsa_lse_f((float)(B + M + K), (float)(B + N + K), T), B, M, N, K, P, T);
+}
 
 // log2 of the modeled time of one contraction, measured H100 model (common.h:138-151).
-TSA_HD float tsa_h100_lt(int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
+TSA_HD float tsa_h100_lt_from(float lab, int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
   if (B + M + N <= P.v2_small_rank) return P.v2_lsmall_cell + (float)(B + M + N + K);
-  const float la = (float)(B + M + K), lb = (float)(B + N + K), lc = (float)(B + M + N);
-  const float lab = tsa_lse_f(la, lb, T), lmoved = tsa_lse_f(lab, lc, T);
+  const float lc = (float)(B + M + N);
+  const float lmoved = tsa_lse_f(lab, lc, T);
   const float perm = P.v2_lperm2 + lab;
   float best = tsa_lse_f(P.v2_lcc_bit + lmoved, P.v2_lcc_cell + (float)(B + M + N + K), T);
   const int MN = M > N ? M : N;
@@ -122,12 +126,40 @@ TSA_HD float tsa_h100_lt(int B, int M, int N, int K, const TsaModel& P, const Ts
   return tsa_lse_f(tsa_lse_f(P.v2_l3launch, perm, T), best, T);
 }
 
+TSA_HD float tsa_h100_lt(int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
+  return tsa_h100_lt_from(tsa_lse_f((float)(B + M + K), (float)(B + N + K), T), B, M, N, K, P, T);
+}
+
 // Cost (log2) of contraction (x, y) -> z with counts B=|xyz|, M=|x~yz|, N=|~xyz|, K=|xy~z|, Z=|z|.
 // Mode 0 is tc = |z| + |x & y & ~z| (common.h:159-163).
 template <int MODE>
 TSA_HD float tsa_node_cost(int B, int M, int N, int K, int Z, const TsaModel& P, const TsaMathTabs& T) {
   if (MODE == 0) return (float)(Z + K);
   return MODE == 1 ? tsa_gpu_lt(B, M, N, K, P, T) : tsa_h100_lt(B, M, N, K, P, T);
+}
+
+// lse_f of two integers: mx + il[mx - mn] with il[d] = log2f(1 + exp2f(-d)), +0 from d = 24 on (where lse_f adds +0
+// too).  exp2f of an integer is exact, so the table holds the floats lse_f itself adds, one look-up instead of the
+// double-precision exponential and logarithm.
+#define TSA_ILSE 32
+TSA_HD float tsa_ilse(int a, int b, const float* il) {
+  const int mx = a > b ? a : b, d = a > b ? a - b : b - a;
+  return (float)mx + il[d < TSA_ILSE - 1 ? d : TSA_ILSE - 1];
+}
+TSA_HD float tsa_ilse_entry(int d, const TsaMathTabs& T) {
+  return d < 24 ? tsa_log2f_12(1.0f + tsa_exp2f_t(-(float)d, T.exp2), T) : 0.0f;
+}
+#if defined(__HIPCC__)
+// The first TSA_ILSE threads of the workgroup fill the table; a workgroup barrier must follow before its use.
+__device__ __forceinline__ void tsa_ilse_stage(float* il, const TsaMathTabs& T) {
+  if (threadIdx.x < TSA_ILSE) il[threadIdx.x] = tsa_ilse_entry((int)threadIdx.x, T);
+}
+#endif
+// tsa_node_cost of the float modes with the operands' sizes folded by table.
+template <int MODE>
+TSA_HD float tsa_node_cost_i(int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T, const float* il) {
+  const float lab = tsa_ilse(B + M + K, B + N + K, il);
+  return MODE == 1 ? tsa_gpu_lt_from(lab, B, M, N, K, P, T) : tsa_h100_lt_from(lab, B, M, N, K, P, T);
 }
 
 // Counters of one proposal: sizes of d (the visited node), P (pivot child) and X (P's new label set),

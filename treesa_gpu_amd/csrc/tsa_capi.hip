@@ -521,6 +521,7 @@ extern "C" int tsa_create(const tsa_layout_t* lay, const uint64_t* leaf, int32_t
     return TSA_ERR_FIT;
   }
   c->Wt = c->L.W;
+  if (use_lds) c->L.team = tsa_team_plan(c->P, nchains, ncu, lds_max, cfg->wide_waves);
   const int leafw = (lay->m * lay->W + 1) & ~1;
   if (cfg->fused_energy) {
     // chains resident at once: workgroups of wpb chains, as many per compute unit as its LDS holds
@@ -558,8 +559,9 @@ extern "C" int tsa_create(const tsa_layout_t* lay, const uint64_t* leaf, int32_t
              lay->W, c->wide.G, c->wide.nsw, c->wide.nt / 64, c->wide.K, c->wide.smem, c->wide.eK, c->wide.fold_stage,
              c->wide.nxcd);
   else
-    snprintf(kb, sizeof kb, "%s W=%d waves/block=%d lds_bytes/wave=%d%s%s", use_lds ? "lds" : "global",
+    snprintf(kb, sizeof kb, "%s W=%d waves/block=%d lds_bytes/wave=%d%s%s%s", use_lds ? "lds" : "global",
              use_lds ? c->Wt : lay->W, c->L.wpb, c->L.lds_words * 8,
+             c->L.team > 0 ? (" par_team_waves=" + std::to_string(c->L.team)).c_str() : "",
              cfg->fused_energy && c->fold_apart ? " fold=apart" : "",
              c->L.draw_waves ? " preorder_draw_waves=3" : "");
   c->kname = kb;
@@ -1968,6 +1970,7 @@ extern "C" int tsa_sweeps_noalloc(const tsa_layout_t* lay, const tsa_config_t* c
   if (plan_one_wave(lay, cfg, nchains, d->lds_max, d->ncu, &L, &in_lds) != TSA_OK) return TSA_ERR_FIT;
   TsaKParams P;
   fill_params(*lay, *cfg, leaf_sc, P);
+  if (in_lds) L.team = tsa_team_plan(P, nchains, d->ncu, d->lds_max, cfg->wide_waves);
   hipStream_t st = static_cast<hipStream_t>(stream);
   unsigned long long* counters = reinterpret_cast<unsigned long long*>(d->scratch);
   float* cost = reinterpret_cast<float*>(d->scratch + kCounterBytes);

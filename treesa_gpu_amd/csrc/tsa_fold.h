@@ -37,36 +37,43 @@ __device__ __forceinline__ float tsa_node_eval(const TsaKParams& P, const uint64
   return tsa_node_cost<MODE>(B, M, N, K, Z, P.model, T);
 }
 
-// The 32-lane fold of cost[0..nint) / z[0..nint) (l32 = lane within a 32-lane group; every lane of the
-// group returns the result).  lf / S / NW serve the masked leaf sizes when S is set.  The lse chain of a
-// lane is serial; its operands are read TSA_FOLD_BATCH at a time ahead of it, so that no step waits on a
-// load, and the size statistics run in a loop of their own.
-// Costs are floats, or (tc mode, whose node costs are integers) 16-bit integers converted exactly.
+// The 32-lane fold of node costs and masked sizes, cost(i) / size(i) for i in [0, nint) (l32 = lane within a
+// 32-lane group; every lane of the group returns the result).  lf / S / NW serve the masked leaf sizes when S is
+// set.  The lse chain of a lane is serial; its operands are read TSA_FOLD_BATCH at a time ahead of it, so that no
+// step waits on a load, and the size statistics run in a loop of their own.
 #define TSA_FOLD_BATCH 8
-template <typename CT>
-__device__ __forceinline__ TsaEvalOut tsa_fold32(const TsaKParams& P, const CT* cost, const uint16_t* z,
-                                                 const uint64_t* S, const uint64_t* lf, int NW, const TsaMathTabs& T,
-                                                 int l32) {
-  const int nint = P.nint, m = P.m;
-  float acc = -INFINITY;
-  for (int i0 = l32; i0 < nint; i0 += 32 * TSA_FOLD_BATCH) {
+// Rows [row0, row1) of the serial part: node 32 * row + l32 of each row folded into acc.
+template <class FC>
+__device__ __forceinline__ float tsa_fold_rows(FC cost, int nint, const TsaMathTabs& T, int l32, float acc, int row0,
+                                               int row1) {
+  const int end = 32 * row1 < nint ? 32 * row1 : nint;
+  for (int i0 = 32 * row0 + l32; i0 < end; i0 += 32 * TSA_FOLD_BATCH) {
     float cb[TSA_FOLD_BATCH];
 #pragma unroll
     for (int q = 0; q < TSA_FOLD_BATCH; q++) {
       const int i = i0 + 32 * q;
-      cb[q] = i < nint ? (float)cost[i] : 0.0f;
+      cb[q] = i < end ? cost(i) : 0.0f;
     }
 #pragma unroll
     for (int q = 0; q < TSA_FOLD_BATCH; q++)
-      if (i0 + 32 * q < nint) acc = tsa_lse_f(acc, cb[q], T);
+      if (i0 + 32 * q < end) acc = tsa_lse_f(acc, cb[q], T);
   }
+  return acc;
+}
+
+// The rest of the fold: the size statistics, then the butterfly over the lanes' acc.
+template <class FZ>
+__device__ __forceinline__ TsaEvalOut tsa_fold_finish(const TsaKParams& P, FZ size, const uint64_t* S,
+                                                      const uint64_t* lf, int NW, const TsaMathTabs& T, int l32,
+                                                      float acc) {
+  const int nint = P.nint, m = P.m;
   int scl = 0, cntl = 0;
   for (int i0 = l32; i0 < nint; i0 += 32 * TSA_FOLD_BATCH) {  // (the sizes read ahead too)
     int zb[TSA_FOLD_BATCH];
 #pragma unroll
     for (int q = 0; q < TSA_FOLD_BATCH; q++) {
       const int i = i0 + 32 * q;
-      zb[q] = i < nint ? (int)z[i] : -1;
+      zb[q] = i < nint ? size(i) : -1;
     }
 #pragma unroll
     for (int q = 0; q < TSA_FOLD_BATCH; q++) {
@@ -113,4 +120,15 @@ __device__ __forceinline__ TsaEvalOut tsa_fold32(const TsaKParams& P, const CT* 
   e.ncand = cnt;
   e.ns = ns;
   return e;
+}
+
+// The whole fold of cost[0..nint) / z[0..nint).  Costs are floats, or (tc mode, whose node costs are integers)
+// 16-bit integers converted exactly.
+template <typename CT>
+__device__ __forceinline__ TsaEvalOut tsa_fold32(const TsaKParams& P, const CT* cost, const uint16_t* z,
+                                                 const uint64_t* S, const uint64_t* lf, int NW, const TsaMathTabs& T,
+                                                 int l32) {
+  const float acc = tsa_fold_rows([&](int i) { return (float)cost[i]; }, P.nint, T, l32, -INFINITY, 0,
+                                  (P.nint + 31) / 32);
+  return tsa_fold_finish(P, [&](int i) { return (int)z[i]; }, S, lf, NW, T, l32, acc);
 }

@@ -263,6 +263,14 @@ hipError_t tsa_launch_sweeps(const TsaLaunch& L, int mode, int order, const TsaK
                              const uint64_t* leaf, const uint32_t* fix, int nchains, float beta, uint32_t sweep0,
                              int nsweeps, unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st,
                              hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res) {
+  // (the team's visits take the costs before a move from a cache whose operands are in slot order, so its model may
+  // not tell left from right: the gpu model does when m0 and n0 differ)
+  if (L.team > 0 && L.lds && order == 0 && eo.blk.n == 0 && (mode != 1 || P.model.m0 == P.model.n0)) {
+    return P.slicing ? tsa_launch_team_sliced(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st,
+                                              e0, e1, lv, res)
+                     : tsa_launch_team(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1,
+                                       lv, res);
+  }
   if (P.slicing)
     return tsa_launch_sweeps_sliced(L, mode, order, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st,
                                     e0, e1, lv, res);
