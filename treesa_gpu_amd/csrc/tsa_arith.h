@@ -109,9 +109,9 @@ TSA_HD float tsa_gpu_lt(int B, int M, int N, int K, const TsaModel& P, const Tsa
   return tsa_gpu_lt_from(tsa_lse_f((float)(B + M + K), (float)(B + N + K), T), B, M, N, K, P, T);
 }
 
-// log2 of the modeled time of one contraction, measured H100 model (common.h:138-151).
+// log2 of the modeled time of one contraction, measured H100 model (common.h:138-151); _from: of one above the small
+// rank.
 TSA_HD float tsa_h100_lt_from(float lab, int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
-  if (B + M + N <= P.v2_small_rank) return P.v2_lsmall_cell + (float)(B + M + N + K);
   const float lc = (float)(B + M + N);
   const float lmoved = tsa_lse_f(lab, lc, T);
   const float perm = P.v2_lperm2 + lab;
@@ -126,7 +126,11 @@ TSA_HD float tsa_h100_lt_from(float lab, int B, int M, int N, int K, const TsaMo
   return tsa_lse_f(tsa_lse_f(P.v2_l3launch, perm, T), best, T);
 }
 
+TSA_HD float tsa_h100_small(int B, int M, int N, int K, const TsaModel& P) {
+  return P.v2_lsmall_cell + (float)(B + M + N + K);
+}
 TSA_HD float tsa_h100_lt(int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T) {
+  if (B + M + N <= P.v2_small_rank) return tsa_h100_small(B, M, N, K, P);
   return tsa_h100_lt_from(tsa_lse_f((float)(B + M + K), (float)(B + N + K), T), B, M, N, K, P, T);
 }
 
@@ -158,6 +162,7 @@ __device__ __forceinline__ void tsa_ilse_stage(float* il, const TsaMathTabs& T) 
 // tsa_node_cost of the float modes with the operands' sizes folded by table.
 template <int MODE>
 TSA_HD float tsa_node_cost_i(int B, int M, int N, int K, const TsaModel& P, const TsaMathTabs& T, const float* il) {
+  if (MODE == 2 && B + M + N <= P.v2_small_rank) return tsa_h100_small(B, M, N, K, P);
   const float lab = tsa_ilse(B + M + K, B + N + K, il);
   return MODE == 1 ? tsa_gpu_lt_from(lab, B, M, N, K, P, T) : tsa_h100_lt_from(lab, B, M, N, K, P, T);
 }

@@ -521,7 +521,7 @@ extern "C" int tsa_create(const tsa_layout_t* lay, const uint64_t* leaf, int32_t
     return TSA_ERR_FIT;
   }
   c->Wt = c->L.W;
-  if (use_lds) c->L.team = tsa_team_plan(c->P, nchains, ncu, lds_max, cfg->wide_waves);
+  if (use_lds) c->L.team = tsa_team_plan(c->P, nchains, ncu, lds_max, cfg->wide_waves, &c->L.team_full);
   const int leafw = (lay->m * lay->W + 1) & ~1;
   if (cfg->fused_energy) {
     // chains resident at once: workgroups of wpb chains, as many per compute unit as its LDS holds
@@ -1970,7 +1970,7 @@ extern "C" int tsa_sweeps_noalloc(const tsa_layout_t* lay, const tsa_config_t* c
   if (plan_one_wave(lay, cfg, nchains, d->lds_max, d->ncu, &L, &in_lds) != TSA_OK) return TSA_ERR_FIT;
   TsaKParams P;
   fill_params(*lay, *cfg, leaf_sc, P);
-  if (in_lds) L.team = tsa_team_plan(P, nchains, d->ncu, d->lds_max, cfg->wide_waves);
+  if (in_lds) L.team = tsa_team_plan(P, nchains, d->ncu, d->lds_max, cfg->wide_waves, &L.team_full);
   hipStream_t st = static_cast<hipStream_t>(stream);
   unsigned long long* counters = reinterpret_cast<unsigned long long*>(d->scratch);
   float* cost = reinterpret_cast<float*>(d->scratch + kCounterBytes);

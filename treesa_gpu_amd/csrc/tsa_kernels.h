@@ -36,8 +36,32 @@ enum { TSA_ST_CHUNKS = TSA_NSTAT, TSA_ST_XCHUNKS, TSA_NSTAT_ALL };
 // of waves do not serialize their atomics on one address; the host sums the slots.
 #define TSA_STAT_SLOTS 64
 
-// Words (64-bit) of per-wave LDS for the node arrays: pri, par, work list, uint16 per internal node.
-static inline int tsa_node_words(int nint) { return (3 * ((nint + 3) & ~3) * 2 + 7) / 8; }
+// The par scan.  Node v is active when its priority is nonzero (not yet visited) and its key (priority, id) beats
+// those of its unvisited parent and internal children.  A visited node's priority is 0, so its key is below every
+// unvisited one's and needs no test of its own.  The priorities have TSA_PRI_PAD leading slots, the last of them 0:
+// pri points past them, and a leaf (or the root's parent, for which par holds leaf id 0) is looked up there by a
+// saturating subtraction.  So a lane's test is three look-ups, two three-way maxima and a comparison, with no branch
+// (the short-circuited form of it took some 60 instructions a group, a dozen of them branches).
+#define TSA_PRI_PAD 4
+__device__ __forceinline__ uint32_t tsa_pri_key(const uint16_t* pri, uint32_t m1, uint32_t node) {  // m1 = m - 1
+  return ((uint32_t)pri[(int)__builtin_elementwise_sub_sat(node, m1) - 1] << 16) | node;
+}
+__device__ __forceinline__ uint32_t tsa_max3(uint32_t a, uint32_t b, uint32_t c) {
+  const uint32_t x = a > b ? a : b;
+  return x > c ? x : c;
+}
+// Of node v: pv its priority, kp / kl / kr the keys of its parent and children.
+__device__ __forceinline__ bool tsa_scan_active(uint32_t v, uint32_t pv, uint32_t kp, uint32_t kl, uint32_t kr) {
+  return ((pv << 16) | v) > tsa_max3(tsa_max3(kp, kl, kr), 0xFFFFu, 0u);
+}
+// Set bits of b below this lane.
+__device__ __forceinline__ int tsa_rank(uint64_t b) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+}
+
+// Words (64-bit) of per-wave LDS for the node arrays: pri (with its leading slots), par, work list, uint16 per
+// internal node.
+static inline int tsa_node_words(int nint) { return ((3 * ((nint + 3) & ~3) + TSA_PRI_PAD) * 2 + 7) / 8; }
 
 struct TsaLaunch {
   int W;             // template width: 1, 2, 4, 8, or 0 = runtime width
@@ -46,6 +70,7 @@ struct TsaLaunch {
   int lds_words;     // LDS words per wave
   int draw_waves;    // 1: pre-order sweeps run one chain per workgroup with helper waves that draw ahead
   int lds_max;       // dynamic LDS bytes a workgroup may have, less the kernel's static LDS
+  int team_full;     // k_team's long work-list entries
   int team;          // par sweeps of a chain in LDS: waves per chain of k_team (0: k_sweep, one wave per chain)
 };
 
@@ -158,18 +183,27 @@ hipError_t tsa_launch_sweeps_sliced(const TsaLaunch& L, int mode, int order, con
                                     const uint64_t* leaf, const uint32_t* fix, int nchains, float beta, uint32_t sweep0,
                                     int nsweeps, unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st,
                                     hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res);
-// Par sweeps with L.team waves per chain (tsa_team.h), and the slicing variants; res as above.
-hipError_t tsa_launch_team(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
-                           const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
-                           unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
-                           hipEvent_t e1, const TsaLevels* lv, int* res);
-hipError_t tsa_launch_team_sliced(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec,
-                                  const uint64_t* leaf, const uint32_t* fix, int nchains, float beta, uint32_t sweep0,
-                                  int nsweeps, unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st,
-                                  hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res);
+// Par sweeps with L.team waves per chain (tsa_team.h): work-list entries long (L.team_full) or short, without and with
+// slicing; res as above.
+hipError_t tsa_launch_team_full(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
+                                const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
+                                unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
+                                hipEvent_t e1, const TsaLevels* lv, int* res);
+hipError_t tsa_launch_team_compact(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
+                                   const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
+                                   unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
+                                   hipEvent_t e1, const TsaLevels* lv, int* res);
+hipError_t tsa_launch_team_sliced_full(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
+                                       const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
+                                       unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
+                                       hipEvent_t e1, const TsaLevels* lv, int* res);
+hipError_t tsa_launch_team_sliced_compact(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
+                                          const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
+                                          unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
+                                          hipEvent_t e1, const TsaLevels* lv, int* res);
 // Waves per chain for a par sweep of nchains chains with lds_max bytes of LDS per workgroup (0: k_sweep's one).  want:
-// 0 automatic, 1 one wave, 2..8 that many.
-int tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want);
+// 0 automatic, 1 one wave, 2..8 that many; *full: whether its work-list entries carry the node's words.
+int tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, int* full);
 hipError_t tsa_launch_energy(int Wt, int mode, const TsaKParams& P, const uint64_t* rec, const uint64_t* leaf,
                              const uint32_t* fix, int nchains, float* lc, int* sc, int* ns, hipStream_t st);
 // The fold of node costs a sweep launch left in cost / z (nchains * nint4 each) into lc / sc / ns.
@@ -361,7 +395,7 @@ __host__ __device__ static inline TsaWideLds tsa_wide_lds(int nint, int band, in
   L.dw = b;     b += band ? nint4 * 4 : 0;
   L.sum = b;    b += nint4 * nsw * 8;
   L.lsum = b;   b += mlds * nsw * 8;
-  L.pri = b;    b += nint4 * 2;
+  L.pri = b;    b += (nint4 + TSA_PRI_PAD) * 2;
   L.par = b;    b += nint4 * 2;
   L.wl = b;     b += nint4 * 2;
   L.out = b;    b += coop ? 0 : nint4;

@@ -540,7 +540,7 @@ __device__ __forceinline__ void tsa_level_keep(const TsaLevels& Lv, const TsaKPa
   for (int i = tid; i < Lv.cand_words; i += nthr) d[i] = s[i];
 }
 
-// Parent of every internal node from the children words (the root's is 0xFFFF), by one wave.
+// Parent of every internal node from the children words (the root's: leaf id 0, see tsa_pri_key), by one wave.
 __device__ __forceinline__ void tsa_par_from_children(const uint32_t* ch, uint16_t* par, int nint, int m, int lane) {
   for (int i = lane; i < nint; i += 64) {
     const uint32_t cw = ch[i];
@@ -548,7 +548,7 @@ __device__ __forceinline__ void tsa_par_from_children(const uint32_t* ch, uint16
     if (l >= m) par[l - m] = (uint16_t)(m + i);
     if (r >= m) par[r - m] = (uint16_t)(m + i);
   }
-  if (lane == 0) par[nint - 1] = 0xFFFFu;
+  if (lane == 0) par[nint - 1] = 0u;
 }
 
 // An evaluated level's end for a chain swept by one wave: node costs into the node arrays (pri and par hold
@@ -561,7 +561,7 @@ __device__ __forceinline__ TsaOwn tsa_level_wave(const TsaKParams& P, const TsaL
                                               int c, int ev, int level, TsaOwn o, int lane) {
   const int NW = W > 0 ? W : P.W;
   tsa_wave_sync();
-  float* const ncost = reinterpret_cast<float*>(pri);
+  float* const ncost = reinterpret_cast<float*>(pri);  // (TSA_PRI_PAD uint16 past an 8-byte boundary: aligned)
   for (int i = lane; i < P.nint; i += 64) {
     int Z;
     ncost[i] = tsa_node_eval<W, MODE>(P, lab, ch, Sm, lf, T, i, Z);
@@ -659,8 +659,8 @@ __global__ void __launch_bounds__(256, (LVL && ORDER == 0 && MODE == 0) ? 3 : 1)
   uint64_t* const S = base + P.s_off;
   const bool slicing = SLICE && P.slicing;  // (launched with SLICE only when P.slicing is set)
   const uint64_t* const Sm = slicing ? S : nullptr;
-  uint16_t* const pri = nodes;
-  uint16_t* const par = nodes + nint4;
+  uint16_t* const pri = nodes + TSA_PRI_PAD;
+  uint16_t* const par = pri + nint4;
   uint16_t* const wl = par + nint4;
   uint32_t* const dw = reinterpret_cast<uint32_t*>(wl + nint4);
   int np = 0, na = 0, nst = 0, nv = 0, nsp = 0, nsa = 0, nbusy = 0;
@@ -701,10 +701,11 @@ __global__ void __launch_bounds__(256, (LVL && ORDER == 0 && MODE == 0) ? 3 : 1)
       const uint32_t sw = sweep0 + (uint32_t)s;
       const uint32_t hs = tsa_sweep_hash(sw, (uint32_t)c, P.key0);
       for (int i = lane; i < nint; i += 64) pri[i] = (uint16_t)tsa_par_pri((uint32_t)(m + i), hs);
+      if (lane == 0) pri[-1] = 0;
       if (P.par_band > 0) {
         // depth at sweep start by pointer jumping on (depth << 16 | ancestor) words; an update that reads
         // an already advanced ancestor word still keeps depth(v) = d + depth(ancestor)
-        for (int i = lane; i < nint; i += 64) dw[i] = par[i] == 0xFFFFu ? 0xFFFFu : (0x10000u | par[i]);
+        for (int i = lane; i < nint; i += 64) dw[i] = par[i] < m ? 0xFFFFu : (0x10000u | par[i]);
         tsa_wave_sync();
         for (;;) {
           bool any = false;
@@ -741,14 +742,12 @@ __global__ void __launch_bounds__(256, (LVL && ORDER == 0 && MODE == 0) ? 3 : 1)
       }
       for (;;) {
         if (unvisited == 0) break;
-        // scan: the phase's independent set into the work list.  Node v is active when its priority is
-        // nonzero and its (priority, id) key beats those of its unvisited parent and internal children.
-        // TSA_SCAN_GROUPS 64-entry groups at a time, branch-free: every lane reads its node (from the list),
-        // the node's priority, parent and children words, then the three neighbour priorities (index 0
-        // where there is no such neighbour), so a batch costs two (three with the list) dependent LDS round
-        // trips.
+        // scan: the phase's independent set into the work list (tsa_scan_active).  TSA_SCAN_GROUPS 64-entry groups
+        // at a time: every lane reads its node (from the list), the node's priority, parent and children words, then
+        // the three neighbour priorities, so a batch costs two (three with the list) dependent LDS round trips.
         const int total = shrink ? unvisited : nint;  // entries to scan
         const int ubase = nint4 - unvisited;          // the list's first entry
+        const uint32_t m1 = (uint32_t)m - 1u;
         int cnt = 0, kept = 0;
         for (int i0 = 0; i0 < total; i0 += 64 * TSA_SCAN_GROUPS) {
           const int ng = (total - i0 + 63) >> 6;  // groups present in this batch (wave-uniform)
@@ -758,11 +757,11 @@ __global__ void __launch_bounds__(256, (LVL && ORDER == 0 && MODE == 0) ? 3 : 1)
           for (int q = 0; q < TSA_SCAN_GROUPS; q++) {
             ni[q] = 0;
             pv[q] = 0u;
-            pw[q] = 0xFFFFu;
+            pw[q] = 0u;
             cw[q] = 0u;
             if (q < ng) {
               const int j = i0 + 64 * q + lane;
-              const int jj = j < total ? j : 0;
+              const int jj = j < total ? j : total - 1;
               const int ii = shrink ? (int)wl[ubase + jj] - m : jj;
               ni[q] = ii;
               pv[q] = pri[ii];
@@ -770,35 +769,28 @@ __global__ void __launch_bounds__(256, (LVL && ORDER == 0 && MODE == 0) ? 3 : 1)
               cw[q] = ch[ii];
             }
           }
-          uint32_t np_[TSA_SCAN_GROUPS], nl[TSA_SCAN_GROUPS], nr[TSA_SCAN_GROUPS];
+          uint32_t kp[TSA_SCAN_GROUPS], kl[TSA_SCAN_GROUPS], kr[TSA_SCAN_GROUPS];
 #pragma unroll
           for (int q = 0; q < TSA_SCAN_GROUPS; q++) {
-            np_[q] = nl[q] = nr[q] = 0u;
+            kp[q] = kl[q] = kr[q] = 0u;
             if (q < ng) {
-              const uint32_t p = pw[q], l = cw[q] & 0xFFFFu, r = cw[q] >> 16;
-              np_[q] = pri[p != 0xFFFFu ? p - (uint32_t)m : 0u];
-              nl[q] = pri[l >= (uint32_t)m ? l - (uint32_t)m : 0u];
-              nr[q] = pri[r >= (uint32_t)m ? r - (uint32_t)m : 0u];
+              kp[q] = tsa_pri_key(pri, m1, pw[q]);
+              kl[q] = tsa_pri_key(pri, m1, cw[q] & 0xFFFFu);
+              kr[q] = tsa_pri_key(pri, m1, cw[q] >> 16);
             }
           }
 #pragma unroll
           for (int q = 0; q < TSA_SCAN_GROUPS; q++) {
             if (q >= ng) break;
-            const bool valid = i0 + 64 * q + lane < total;
             const uint32_t v = (uint32_t)(m + ni[q]);
-            const uint32_t key = (pv[q] << 16) | v;
-            const uint32_t p = pw[q], l = cw[q] & 0xFFFFu, r = cw[q] >> 16;
-            const bool beat_p = p != 0xFFFFu && np_[q] != 0u && ((np_[q] << 16) | p) > key;
-            const bool beat_l = l >= (uint32_t)m && nl[q] != 0u && ((nl[q] << 16) | l) > key;
-            const bool beat_r = r >= (uint32_t)m && nr[q] != 0u && ((nr[q] << 16) | r) > key;
-            const bool act = valid && pv[q] != 0u && !beat_p && !beat_l && !beat_r;
-            const uint64_t b = __ballot(act);
-            if (act) wl[cnt + __popcll(b & tsa_lt_mask(lane))] = (uint16_t)v;
+            const int left_here = total - (i0 + 64 * q);  // entries from this group on
+            const uint64_t vm = left_here >= 64 ? ~0ull : (1ull << left_here) - 1ull;
+            const uint64_t b = __ballot(tsa_scan_active(v, pv[q], kp[q], kl[q], kr[q])) & vm;
+            if ((b >> lane) & 1ull) wl[cnt + tsa_rank(b)] = (uint16_t)v;
             cnt += __popcll(b);
             if (shrink) {
-              const bool keep = valid && !act;
-              const uint64_t bk = __ballot(keep);
-              if (keep) wl[nint4 - 1 - (kept + __popcll(bk & tsa_lt_mask(lane)))] = (uint16_t)v;
+              const uint64_t bk = vm & ~b;
+              if ((bk >> lane) & 1ull) wl[nint4 - 1 - (kept + tsa_rank(bk))] = (uint16_t)v;
               kept += __popcll(bk);
             }
           }

@@ -18,32 +18,34 @@
 // The phases, draws, floats and counters are those of the one-wave kernel (and of the CPU phase-by-phase sweep) bit
 // for bit; visits of one phase touch disjoint words, so their order is free.
 //
-// Included by two translation units, one per SLICE variant.
+// Included by four translation units, one per SLICE and FULL variant.
 #pragma once
 #include "tsa_sweep.h"
 
-// LDS byte offsets (same function on host and device): leaf sets ending where the record starts, the record, the
-// node arrays, two buffers of draws, then `caches` copies of the node-cost cache.
+// LDS byte offsets (same function on host and device): leaf sets ending where the record starts, the record, the work
+// list, two buffers of draws, `caches` copies of the node-cost cache, then the node arrays.  A work-list entry is the
+// node's children word, draw and cost word and its id (full: a visit then starts with the pivot's children word, two
+// dependent LDS round trips earlier), or the id alone.
 struct TsaTeamLds {
-  int leaf, rec, pri, par, wl, draw, cache, cache_bytes, bytes;
+  int leaf, rec, wl, draw, cache, cache_bytes, nodes, bytes;
 };
 __host__ __device__ static inline TsaTeamLds tsa_team_lds(int m, int nint, int W, int chain_words, int mode,
-                                                          int caches) {
+                                                          int caches, int full) {
   const int nint4 = (nint + 3) & ~3, leafb = (m * W * 8 + 15) & ~15;
   TsaTeamLds L;
   L.leaf = leafb - m * W * 8;
   int b = leafb;
   L.rec = b;   b += chain_words * 8;
+  L.wl = b;    b += nint4 * (full ? 16 : 2);
   L.draw = b;  b += 2 * nint4 * 4;
   L.cache = b;
   L.cache_bytes = nint4 * (mode == 0 ? 4 : 6);
   b += caches * L.cache_bytes;
-  L.pri = b;   b += nint4 * 2;
-  L.par = b;   b += nint4 * 2;
-  L.wl = b;    b += nint4 * 2;
+  L.nodes = b; b += (2 * nint4 + TSA_PRI_PAD) * 2;  // priorities, parents
   L.bytes = (b + 15) & ~15;
   return L;
 }
+#define TSA_TEAM_STATIC_LDS 4096  // room for k_team's static LDS (under 3.5 KB)
 // Copies of the cache a launch needs: the chain's, the proposed slice set's, and the level being folded.
 static inline int tsa_team_caches(bool slice_moves, bool levels) { return 1 + (slice_moves ? 1 : 0) + (levels ? 1 : 0); }
 
@@ -239,7 +241,7 @@ __device__ __attribute__((noinline)) TsaOwn tsa_team_fold_end(const TsaTeamFold*
   return tsa_level_arrive(F->Lv, F->n, F->c, ev, level, e.lcost, e.sc, e.ns, own, slot, lane);
 }
 
-template <int W, int MODE, bool SLICE, bool LVL>
+template <int W, int MODE, bool SLICE, bool LVL, bool FULL>
 __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
     k_team(TsaKParams P, uint64_t* __restrict__ rec, const uint64_t* __restrict__ leaf,
            const uint32_t* __restrict__ fix, int nchains, float beta1, uint32_t sweep0, int nsweeps,
@@ -256,7 +258,8 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
   const int m = P.m, nint = P.nint, ngrp = (nint + 63) >> 6;
   const int c = P.chain0 + (int)blockIdx.x;  // (the grid is nchains - chain0 workgroups)
   const bool moves = SLICE && P.slice_moves > 0;
-  const TsaTeamLds Lo = tsa_team_lds(m, nint, W, P.chain_words, MODE, 1);
+  const int ncache = 1 + (moves ? 1 : 0) + (LVL ? 1 : 0);
+  const TsaTeamLds Lo = tsa_team_lds(m, nint, W, P.chain_words, MODE, ncache, FULL);
   uint64_t* const lf = reinterpret_cast<uint64_t*>(tsa_tsm + Lo.leaf);
   uint64_t* const base = reinterpret_cast<uint64_t*>(tsa_tsm + Lo.rec);
   uint64_t* const lab = base;
@@ -265,15 +268,14 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
   const uint64_t* const Sm = SLICE ? S : nullptr;
   uint32_t* const draws = reinterpret_cast<uint32_t*>(tsa_tsm + Lo.draw);
   const int nint4 = (nint + 3) & ~3;
-  const int cb = Lo.cache_bytes, ncache = 1 + (moves ? 1 : 0) + (LVL ? 1 : 0);
   auto cache_at = [&](int k) {
-    unsigned char* const p = tsa_tsm + Lo.cache + k * cb;
+    unsigned char* const p = tsa_tsm + Lo.cache + k * Lo.cache_bytes;
     return TsaTeamCache<MODE>{reinterpret_cast<uint32_t*>(p), reinterpret_cast<uint16_t*>(p + nint4 * 4)};
   };
-  unsigned char* const nodes = tsa_tsm + Lo.cache + ncache * cb;
-  uint16_t* const pri = reinterpret_cast<uint16_t*>(nodes);
+  uint16_t* const pri = reinterpret_cast<uint16_t*>(tsa_tsm + Lo.nodes) + TSA_PRI_PAD;
   uint16_t* const par = pri + nint4;
-  uint16_t* const wl = par + nint4;
+  uint4* const wl4 = reinterpret_cast<uint4*>(tsa_tsm + Lo.wl);       // FULL
+  uint16_t* const wl = reinterpret_cast<uint16_t*>(tsa_tsm + Lo.wl);  // else
   TsaTeamCache<MODE> cc = cache_at(0);
   TsaTeamCache<MODE> cprop = cache_at(moves ? 1 : 0);         // the proposed slice set's costs
   const TsaTeamCache<MODE> cfold = cache_at(ncache - 1);      // LVL: the level being folded
@@ -317,7 +319,10 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
     const float cst = tsa_node_eval<W, MODE>(P, lab, ch, Sm, lf, T_, i, Z);
     cc.set(i, cst, Z);
   }
-  if (tid == 0) par[nint - 1] = 0xFFFFu;
+  if (tid == 0) {
+    par[nint - 1] = 0u;  // (leaf id 0: no parent, see tsa_pri_key)
+    pri[-1] = 0;
+  }
 
   // the level loop: the last wave tracks the chain; its fold of an evaluated level runs a few rows per phase of
   // the sweeps that follow (frow: the next row, -1 none)
@@ -376,57 +381,63 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
     };
     bool draws_left = draw_next;
     int unvisited = nint;
+    const uint32_t m1 = (uint32_t)m - 1u;
     while (unvisited > 0) {
       // scan: this wave's groups, TSA_TEAM_SCAN at a time (every read of a batch in flight at once)
       for (int g0 = wv; g0 < ngrp; g0 += T * TSA_TEAM_SCAN) {
-        uint32_t pv[TSA_TEAM_SCAN], pw[TSA_TEAM_SCAN], cw[TSA_TEAM_SCAN];
-        uint32_t np_[TSA_TEAM_SCAN], nl[TSA_TEAM_SCAN], nr[TSA_TEAM_SCAN];
+        uint32_t pv[TSA_TEAM_SCAN], pw[TSA_TEAM_SCAN], kp[TSA_TEAM_SCAN], kl[TSA_TEAM_SCAN], kr[TSA_TEAM_SCAN];
+        uint4 en[TSA_TEAM_SCAN];
 #pragma unroll
         for (int q = 0; q < TSA_TEAM_SCAN; q++) {
           const int gi = g0 + q * T;
-          pv[q] = 0u;
-          pw[q] = 0xFFFFu;
-          cw[q] = 0u;
+          pv[q] = pw[q] = 0u;
+          en[q] = uint4{0u, 0u, 0u, 0u};
           if (gi < ngrp) {  // uniform
             const int i = gi * 64 + lane, ic = i < nint ? i : nint - 1;
-            pv[q] = i < nint ? pri[ic] : 0u;
+            pv[q] = pri[ic];
             pw[q] = par[ic];
-            cw[q] = ch[ic];
+            en[q] = uint4{ch[ic], 0u, 0u, (uint32_t)(m + ic)};
+            if constexpr (FULL) {
+              en[q].y = dr[ic];
+              en[q].z = cc.a[ic];
+            }
           }
         }
 #pragma unroll
         for (int q = 0; q < TSA_TEAM_SCAN; q++) {
-          np_[q] = nl[q] = nr[q] = 0u;
+          kp[q] = kl[q] = kr[q] = 0u;
           if (g0 + q * T < ngrp) {
-            const uint32_t p = pw[q], l = cw[q] & 0xFFFFu, r = cw[q] >> 16;
-            np_[q] = pri[p != 0xFFFFu ? p - (uint32_t)m : 0u];
-            nl[q] = pri[l >= (uint32_t)m ? l - (uint32_t)m : 0u];
-            nr[q] = pri[r >= (uint32_t)m ? r - (uint32_t)m : 0u];
+            kp[q] = tsa_pri_key(pri, m1, pw[q]);
+            kl[q] = tsa_pri_key(pri, m1, en[q].x & 0xFFFFu);
+            kr[q] = tsa_pri_key(pri, m1, en[q].x >> 16);
           }
         }
         uint64_t bb[TSA_TEAM_SCAN];
         int tot = 0;
 #pragma unroll
         for (int q = 0; q < TSA_TEAM_SCAN; q++) {
-          const uint32_t v = (uint32_t)(m + (g0 + q * T) * 64 + lane), key = (pv[q] << 16) | v;
-          const uint32_t p = pw[q], l = cw[q] & 0xFFFFu, r = cw[q] >> 16;
-          const bool beat_p = p != 0xFFFFu && np_[q] != 0u && ((np_[q] << 16) | p) > key;
-          const bool beat_l = l >= (uint32_t)m && nl[q] != 0u && ((nl[q] << 16) | l) > key;
-          const bool beat_r = r >= (uint32_t)m && nr[q] != 0u && ((nr[q] << 16) | r) > key;
-          bb[q] = __ballot(pv[q] != 0u && !beat_p && !beat_l && !beat_r);
+          const int here = nint - (g0 + q * T) * 64;  // nodes from this group on
+          const uint64_t vm = here >= 64 ? ~0ull : here > 0 ? (1ull << here) - 1ull : 0ull;
+          bb[q] = __ballot(tsa_scan_active(en[q].w, pv[q], kp[q], kl[q], kr[q])) & vm;
           tot += __popcll(bb[q]);
         }
+        if (tot == 0) continue;
         int at = 0;
-        if (lane == 0 && tot) at = atomicAdd(&s_cnt[ph & 1], tot);
+        if (lane == 0) at = atomicAdd(&s_cnt[ph & 1], tot);
         at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
         for (int q = 0; q < TSA_TEAM_SCAN; q++) {
-          if ((bb[q] >> lane) & 1ull)
-            wl[at + __popcll(bb[q] & tsa_lt_mask(lane))] = (uint16_t)(m + (g0 + q * T) * 64 + lane);
+          if ((bb[q] >> lane) & 1ull) {
+            if constexpr (FULL) wl4[at + tsa_rank(bb[q])] = en[q];
+            else wl[at + tsa_rank(bb[q])] = (uint16_t)en[q].w;
+          }
           at += __popcll(bb[q]);
         }
       }
       __syncthreads();
+      const int j0 = wv * GPW;
+      uint4 w{};
+      if constexpr (FULL) w = wl4[j0 + gsub < nint4 ? j0 + gsub : 0];  // (beside the count; used when there is such an entry)
       const int cnt = s_cnt[ph & 1];
       if (cnt == 0) break;  // (uniform; only a record that holds no tree)
       if (tid == 0) s_cnt[(ph + 1) & 1] = 0;  // (last read before the previous phase's second barrier)
@@ -442,17 +453,25 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
           fold_end();
         }
       }
-      const int j0 = wv * GPW;
       if (j0 >= cnt && draws_left) draws_left = draw_some();
       for (int j1 = j0; j1 < cnt; j1 += T * GPW) {
         const int j = j1 + gsub;
         if (j >= cnt) continue;  // whole groups
-        const int v = wl[j], vi = v - m;
-        const uint32_t chv = ch[vi], d = dr[vi];
+        if constexpr (!FULL) {
+          w.w = wl[j];
+          const int i = (int)w.w - m;
+          w.x = ch[i];
+          w.y = dr[i];
+          w.z = cc.a[i];
+        } else if (j1 > j0) {
+          w = wl4[j];
+        }
+        const int v = (int)w.w, vi = v - m;
+        const uint32_t chv = w.x, d = w.y;
         const int l = (int)(chv & 0xFFFFu), r = (int)(chv >> 16);
         const bool li = l >= m, ri = r >= m;
         if (li || ri) {
-          const float costV = cc.cost(vi);
+          const float costV = MODE == 0 ? (float)(w.z & 0xFFFFu) : __uint_as_float(w.z);
           const int b2 = (int)(d & 3u);
           const int rule = li && ri ? b2 : (li ? b2 >> 1 : 2 + (b2 >> 1));
           const int slotP = tsa_slot_p(rule), slotM = tsa_slot_m(rule);
@@ -561,7 +580,7 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
     }
     if constexpr (LVL) {
       if (--left == 0) {  // the level's last sweep
-        const int ev = Lv.eval[lv];
+        const int ev = F->Lv.eval[lv];
         if (ev >= 0) {
           if (tracker && frow >= 0) fold_end();  // the previous level's, not yet done
           __syncthreads();
@@ -572,16 +591,16 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
           if (SLICE && tid < W) s_S[tid] = S[tid];
           if (tracker) {
             fslot = own.slot < 0 ? 0 : own.slot ^ 1;
-            tsa_level_keep(Lv, P, base, nchains, c, fslot, lane, 64);
+            tsa_level_keep(F->Lv, P, base, nchains, c, fslot, lane, 64);
             frow = 0;
             facc = -INFINITY;
             fev = ev;
             flev = lv;
           }
         }
-        if (++lv < Lv.nlev) {
-          beta = Lv.beta[lv];
-          left = Lv.niters[lv];
+        if (++lv < F->Lv.nlev) {
+          beta = F->Lv.beta[lv];
+          left = F->Lv.niters[lv];
         }
       }
     }
@@ -591,8 +610,8 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
     if (tracker) {
       if (frow >= 0) fold_end();
       if (lane == 0) {
-        Lv.own[c] = own.s;
-        Lv.bslot[c] = own.slot;
+        F->Lv.own[c] = own.s;
+        F->Lv.bslot[c] = own.slot;
       }
     }
   }
@@ -638,52 +657,52 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
   }
 }
 
-template <int W, int MODE, bool SLICE, bool LVL>
+template <int W, int MODE, bool SLICE, bool LVL, bool FULL>
 static hipError_t launch_team_t(const TsaLaunch& L, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
                                 const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
                                 unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
                                 hipEvent_t e1, const TsaLevels* lv, int* res) {
   const int caches = tsa_team_caches(SLICE && P.slice_moves > 0, LVL);
-  const size_t smem = (size_t)tsa_team_lds(P.m, P.nint, W, P.chain_words, MODE, caches).bytes;
+  const size_t smem = (size_t)tsa_team_lds(P.m, P.nint, W, P.chain_words, MODE, caches, FULL).bytes;
   const int threads = 64 * L.team;
-  const void* const fn = reinterpret_cast<const void*>(&k_team<W, MODE, SLICE, LVL>);
+  const void* const fn = reinterpret_cast<const void*>(&k_team<W, MODE, SLICE, LVL, FULL>);
   if (smem > 65536) {
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return e;
   }
   if (res) return hipOccupancyMaxActiveBlocksPerMultiprocessor(res, fn, threads, smem);  // a query, no launch
   if (P.chain0 < 0 || P.chain0 >= nchains) return hipErrorInvalidValue;
-  hipExtLaunchKernelGGL((k_team<W, MODE, SLICE, LVL>), dim3(nchains - P.chain0), dim3(threads), (uint32_t)smem, st, e0,
+  hipExtLaunchKernelGGL((k_team<W, MODE, SLICE, LVL, FULL>), dim3(nchains - P.chain0), dim3(threads), (uint32_t)smem, st, e0,
                         e1, 0u, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, lv ? *lv : TsaLevels{});
   return hipGetLastError();
 }
 
-template <int W, bool SLICE>
+template <int W, bool SLICE, bool FULL>
 static hipError_t launch_team_w(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
                                 const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
                                 unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
                                 hipEvent_t e1, const TsaLevels* lv, int* res) {
 #define TSA_TEAM_GO(MODE)                                                                                              \
-  return lv ? launch_team_t<W, MODE, SLICE, true>(L, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, \
-                                                  e0, e1, lv, res)                                                     \
-            : launch_team_t<W, MODE, SLICE, false>(L, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo,    \
-                                                   st, e0, e1, lv, res)
+  return lv ? launch_team_t<W, MODE, SLICE, true, FULL>(L, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats,   \
+                                                        eo, st, e0, e1, lv, res)                                       \
+            : launch_team_t<W, MODE, SLICE, false, FULL>(L, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats,  \
+                                                         eo, st, e0, e1, lv, res)
   if (mode == 0) TSA_TEAM_GO(0);
   if (mode == 1) TSA_TEAM_GO(1);
   TSA_TEAM_GO(2);
 #undef TSA_TEAM_GO
 }
 
-template <bool SLICE>
+template <bool SLICE, bool FULL>
 static hipError_t tsa_launch_team_t(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec,
                                     const uint64_t* leaf, const uint32_t* fix, int nchains, float beta,
                                     uint32_t sweep0, int nsweeps, unsigned long long* stats, const TsaEnergyOut& eo,
                                     hipStream_t st, hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res) {
   switch (L.W) {
-    case 1: return launch_team_w<1, SLICE>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
-    case 2: return launch_team_w<2, SLICE>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
-    case 4: return launch_team_w<4, SLICE>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
-    case 8: return launch_team_w<8, SLICE>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
+    case 1: return launch_team_w<1, SLICE, FULL>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
+    case 2: return launch_team_w<2, SLICE, FULL>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
+    case 4: return launch_team_w<4, SLICE, FULL>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
+    case 8: return launch_team_w<8, SLICE, FULL>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
     default: return hipErrorInvalidValue;
   }
 }

@@ -1,21 +1,24 @@
-// tsa_team.hip -- the variants of k_team (tsa_team.h) without slicing.
+// tsa_team.hip -- the variants of k_team (tsa_team.h) without slicing, long work-list entries; and the choice of the team.
 #include "tsa_team.h"
 
-hipError_t tsa_launch_team(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
-                           const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
-                           unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
-                           hipEvent_t e1, const TsaLevels* lv, int* res) {
-  return tsa_launch_team_t<false>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv,
-                                  res);
+hipError_t tsa_launch_team_full(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
+                                const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
+                                unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
+                                hipEvent_t e1, const TsaLevels* lv, int* res) {
+  return tsa_launch_team_t<false, true>(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1,
+                                   lv, res);
 }
 
-int tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want) {
+int tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, int* full) {
+  *full = 0;
   if (want == 1 || want > 8 || P.par_follow || P.par_band > 0) return 0;
   // the most LDS any launch of the context asks for: a float mode's cache, the level loop, slice moves
-  const int most = tsa_team_lds(P.m, P.nint, P.W, P.chain_words, 1, tsa_team_caches(P.slicing && P.slice_moves > 0, true)).bytes;
-  if (most > lds_max - 4096) return 0;
-  if (want > 1) return want;
+  const int caches = tsa_team_caches(P.slicing && P.slice_moves > 0, true);
+  if (tsa_team_lds(P.m, P.nint, P.W, P.chain_words, 1, caches, 0).bytes > lds_max - TSA_TEAM_STATIC_LDS) return 0;
   const int per_cu = (nchains + (ncu > 0 ? ncu : 1) - 1) / (ncu > 0 ? ncu : 1);
-  const int T = per_cu <= 2 ? 8 : per_cu <= 4 ? 4 : per_cu <= 8 ? 2 : 0;
-  return T;
+  // long entries save a visit two dependent LDS round trips; they may not cost a compute unit a chain
+  const int most = tsa_team_lds(P.m, P.nint, P.W, P.chain_words, 1, caches, 1).bytes + TSA_TEAM_STATIC_LDS;
+  *full = most <= lds_max && (long long)most * per_cu <= lds_max;
+  if (want > 1) return want;
+  return per_cu <= 2 ? 8 : per_cu <= 4 ? 4 : per_cu <= 8 ? 2 : 0;
 }

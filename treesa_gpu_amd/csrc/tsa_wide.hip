@@ -50,8 +50,6 @@ struct alignas(16) TsaW2 {
   uint64_t a, b;
 };
 
-__device__ __forceinline__ uint64_t wide_lt_mask(int lane) { return (1ull << lane) - 1ull; }
-
 // Counters of one proposal as a flat list: |d|, |P|, |X|, then K0..K3 (mode 0) or B0..3, M0..3, N0..3,
 // K0..3 (modes 1, 2).
 template <int MODE>
@@ -293,7 +291,7 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
   uint64_t* const masks = reinterpret_cast<uint64_t*>(tsa_wsm + Lo.masks);
   uint32_t* const ch = reinterpret_cast<uint32_t*>(tsa_wsm + Lo.ch);
   uint32_t* const dw = reinterpret_cast<uint32_t*>(tsa_wsm + Lo.dw);
-  uint16_t* const pri = reinterpret_cast<uint16_t*>(tsa_wsm + Lo.pri);
+  uint16_t* const pri = reinterpret_cast<uint16_t*>(tsa_wsm + Lo.pri) + TSA_PRI_PAD;
   uint16_t* const par = reinterpret_cast<uint16_t*>(tsa_wsm + Lo.par);
   uint16_t* const wl = reinterpret_cast<uint16_t*>(tsa_wsm + Lo.wl);
   uint8_t* const outl = tsa_wsm + Lo.out;
@@ -317,7 +315,10 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
     if (l >= m) par[l - m] = (uint16_t)(m + i);
     if (r >= m) par[r - m] = (uint16_t)(m + i);
   }
-  if (threadIdx.x == 0) par[nint - 1] = 0xFFFFu;
+  if (threadIdx.x == 0) {
+    par[nint - 1] = 0u;  // (leaf id 0: no parent, see tsa_pri_key)
+    pri[-1] = 0;
+  }
   __syncthreads();
 
   // K > 1: check in (see the file comment); a chain claimed by one workgroup is swept by it alone (Ke = 1)
@@ -357,7 +358,7 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
     if (P.par_band > 0) {
       // depth at sweep start by pointer jumping on (depth << 16 | ancestor) words; an update that reads an
       // already advanced ancestor word still keeps depth(v) = d + depth(ancestor)
-      for (int i = threadIdx.x; i < nint; i += NT) dw[i] = par[i] == 0xFFFFu ? 0xFFFFu : (0x10000u | par[i]);
+      for (int i = threadIdx.x; i < nint; i += NT) dw[i] = par[i] < m ? 0xFFFFu : (0x10000u | par[i]);
       __syncthreads();
       for (;;) {
         int any = 0;
@@ -387,8 +388,8 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
     for (;;) {
       if (!P.par_follow && unvisited == 0) break;  // uniform across the workgroup
       // 1. scan: a wave takes 64-node groups; each lane reads its node's priority, parent and children
-      // words, then the three neighbour priorities, in two rounds of independent LDS reads (indices are
-      // clamped instead of branched on, so that every read of a round is in flight at once)
+      // words, then the three neighbour priorities, in two rounds of independent LDS reads (tsa_scan_active:
+      // no branches, so that every read of a round is in flight at once)
       // a wave takes its groups eight at a time: eight ballots, then (one workgroup per chain) one append
       for (int g0 = wv; g0 < ngrp; g0 += 8 * nwv) {
         uint64_t bb[8];
@@ -398,12 +399,9 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
           const int i = gi * 64 + lane;
           const int ic = i < nint ? i : nint - 1;
           const uint32_t pv = pri[ic], p = par[ic], cw = ch[ic];
-          const uint32_t l = cw & 0xFFFFu, r = cw >> 16;
-          const bool hp = p != 0xFFFFu, hl = l >= (uint32_t)m, hr = r >= (uint32_t)m;
-          const uint32_t pp = pri[hp ? (int)p - m : ic], pl = pri[hl ? (int)l - m : ic], pr = pri[hr ? (int)r - m : ic];
-          const uint32_t key = (pv << 16) | (uint32_t)(m + i);
-          const bool act = gi < ngrp && i < nint && pv != 0u && !(hp && pp && ((pp << 16) | p) > key) &&
-                           !(hl && pl && ((pl << 16) | l) > key) && !(hr && pr && ((pr << 16) | r) > key);
+          const uint32_t kp = tsa_pri_key(pri, (uint32_t)m - 1u, p), kl = tsa_pri_key(pri, (uint32_t)m - 1u, cw & 0xFFFFu),
+                         kr = tsa_pri_key(pri, (uint32_t)m - 1u, cw >> 16);
+          const bool act = tsa_scan_active((uint32_t)(m + ic), pv, kp, kl, kr) & (gi < ngrp) & (i < nint);
           bb[q] = __ballot(act);
           if (COOP && lane == 0 && gi < ngrp) masks[gi] = bb[q];
         }
@@ -419,7 +417,7 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
 #pragma unroll
           for (int q = 0; q < 8; q++) {
             const uint64_t b = bb[q];
-            if ((b >> lane) & 1ull) wl[base + __popcll(b & wide_lt_mask(lane))] = (uint16_t)(m + (g0 + q * nwv) * 64 + lane);
+            if ((b >> lane) & 1ull) wl[base + tsa_rank(b)] = (uint16_t)(m + (g0 + q * nwv) * 64 + lane);
             base += __popcll(b);
           }
         }
@@ -446,7 +444,7 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
             const uint32_t bhi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), gi - g0);
             const uint64_t bm = ((uint64_t)bhi << 32) | blo;
             const int off = __builtin_amdgcn_readlane(excl, gi - g0);
-            if ((bm >> lane) & 1ull) wl[off + __popcll(bm & wide_lt_mask(lane))] = (uint16_t)(m + gi * 64 + lane);
+            if ((bm >> lane) & 1ull) wl[off + tsa_rank(bm)] = (uint16_t)(m + gi * 64 + lane);
           }
           base += __builtin_amdgcn_readlane(y, 63);
         }
