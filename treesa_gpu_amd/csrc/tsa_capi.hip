@@ -130,6 +130,7 @@ struct tsa_ctx {
   bool track_pending[TSA_SNAP_MAX] = {};
   int slot = 0, last_slot = -1;  // slot of the next sweep launch / of the last one (-1: none since a reset)
   int nslots = 0;                // slots allocated (their buffers), the ones in turn
+  std::vector<char*> slot_slabs; // the allocations the slots' buffers lie in, one per ensure_slots that grew them
   uint32_t* d_snap_ch[TSA_SNAP_MAX] = {};
   float* d_snap_cost[TSA_SNAP_MAX] = {};
   uint16_t* d_snap_nz[TSA_SNAP_MAX] = {};
@@ -143,6 +144,7 @@ struct tsa_ctx {
   // dispatch (about 6 us of host time) rather than in the dispatch itself (about 20 us).
   bool host_waited = false;
   int track_kind = 0;
+  bool anneal_blocks = false;  // tsa_anneal ran this session's levels in blocks where it would have run the loop
   bool lv_reset = false;
   int lv_resident[6] = {-1, -1, -1, -1, -1, -1};  // level-loop chains resident per compute unit, per mode and order
   int blocks_k = 0;   // levels per launch of tsa_anneal's last block path (reported by tsa_describe)
@@ -344,11 +346,8 @@ static void free_ctx(tsa_ctx* c) {
   }
   for (int k = 0; k < TSA_SNAP_MAX; k++) {
     if (c->ev_track[k]) (void)hipEventDestroy(c->ev_track[k]);
-    if (c->d_snap_ch[k]) (void)hipFree(c->d_snap_ch[k]);
-    if (c->d_snap_cost[k]) (void)hipFree(c->d_snap_cost[k]);
-    if (c->d_snap_nz[k]) (void)hipFree(c->d_snap_nz[k]);
-    if (c->d_snap_en[k]) (void)hipFree(c->d_snap_en[k]);
   }
+  for (char* p : c->slot_slabs) (void)hipFree(p);
   if (c->ev_tinit) (void)hipEventDestroy(c->ev_tinit);
   if (c->st2) (void)hipStreamDestroy(c->st2);
   if (c->d_track) (void)hipFree(c->d_track);
@@ -521,7 +520,7 @@ extern "C" int tsa_create(const tsa_layout_t* lay, const uint64_t* leaf, int32_t
     return TSA_ERR_FIT;
   }
   c->Wt = c->L.W;
-  if (use_lds) c->L.team = tsa_team_plan(c->P, nchains, ncu, lds_max, cfg->wide_waves, &c->L.team_full);
+  if (use_lds) tsa_team_plan(c->P, nchains, ncu, lds_max, cfg->wide_waves, &c->L);
   const int leafw = (lay->m * lay->W + 1) & ~1;
   if (cfg->fused_energy) {
     // chains resident at once: workgroups of wpb chains, as many per compute unit as its LDS holds
@@ -729,6 +728,13 @@ static bool wide_blocks_ok(const tsa_ctx* c, int order) {
          !c->cfg.slicing && order == TSA_ORDER_PAR;
 }
 
+// Blocks of levels on the one-wave and team kernels: the chain in LDS, par order, the overlapped selection with the
+// node-cost snapshots folded apart (level_loop -1, launches per level, keeps them where a level's fold runs apart).
+static bool lds_blocks_ok(const tsa_ctx* c, int order, int k) {
+  return k > 1 && (c->fold_apart || c->cfg.level_loop >= 0) && c->overlap && !c->wide.on && c->L.lds && c->cfg.fused_energy != 0 && !c->cfg.slicing &&
+         order == TSA_ORDER_PAR;
+}
+
 static hipError_t quiesce_track(tsa_ctx* c) {
   hipError_t e = hipSuccess;
   if (c->st2) e = hipStreamSynchronize(c->st2);
@@ -742,13 +748,21 @@ static hipError_t quiesce_track(tsa_ctx* c) {
 static int ensure_slots(tsa_ctx* ctx, int n) {
   if (n > TSA_SNAP_MAX) return fail(ctx, TSA_ERR_ARG, "snapshot slots: more than TSA_SNAP_MAX");
   const size_t nint = (size_t)ctx->lay.nint, nint4 = (nint + 3) & ~(size_t)3;
-  for (int k = ctx->nslots; k < n; k++) {
-    TSA_HIP(ctx, hipMalloc(&ctx->d_snap_ch[k], (size_t)ctx->nchains * nint * 4));
-    TSA_HIP(ctx, hipMalloc(&ctx->d_snap_cost[k], (size_t)ctx->nchains * nint4 * 4));
-    TSA_HIP(ctx, hipMalloc(&ctx->d_snap_nz[k], (size_t)ctx->nchains * nint4 * 2));
-    TSA_HIP(ctx, hipMalloc(&ctx->d_snap_en[k], (size_t)ctx->nchains * 12));
-    ctx->nslots = k + 1;
+  if (n <= ctx->nslots) return TSA_OK;
+  // one allocation for all of them (a block's 24 slots by four buffers each took a run's first pass milliseconds)
+  const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t nc = (size_t)ctx->nchains, bch = up(nc * nint * 4), bcost = up(nc * nint4 * 4), bnz = up(nc * nint4 * 2),
+               ben = up(nc * 12), slot = bch + bcost + bnz + ben;
+  char* p = nullptr;
+  TSA_HIP(ctx, hipMalloc(&p, (size_t)(n - ctx->nslots) * slot));
+  ctx->slot_slabs.push_back(p);
+  for (int k = ctx->nslots; k < n; k++, p += slot) {
+    ctx->d_snap_ch[k] = reinterpret_cast<uint32_t*>(p);
+    ctx->d_snap_cost[k] = reinterpret_cast<float*>(p + bch);
+    ctx->d_snap_nz[k] = reinterpret_cast<uint16_t*>(p + bch + bcost);
+    ctx->d_snap_en[k] = reinterpret_cast<uint32_t*>(p + bch + bcost + bnz);
   }
+  ctx->nslots = n;
   return TSA_OK;
 }
 
@@ -875,6 +889,11 @@ extern "C" int tsa_wait(tsa_ctx* ctx) {
   return TSA_OK;
 }
 
+// Whether a sweep whose fold runs apart is split over two streams: a block of levels of four chains and more per
+// compute unit (fewer leave compute units idle, and two halves of them only add a launch: 256 chains of sat100 605
+// against 672 us per 40 levels, 1024 935 against 901); a launch of one level of any population that folds apart.
+static bool split_pays(const tsa_ctx* ctx, const TsaBlock* blk) { return !blk || ctx->nchains >= 4 * ctx->ncu; }
+
 // The first chain of a split level's second launch: half the chains, in whole workgroups.
 static int split_point(const tsa_ctx* ctx) {
   return (ctx->nchains / 2 + ctx->L.wpb - 1) / ctx->L.wpb * ctx->L.wpb;
@@ -996,10 +1015,10 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
     ctx->costs_valid = false;
     ctx->sums_valid = false;
     const bool fuse = ctx->cfg.fused_energy != 0;
-    const bool apart = fuse && ctx->fold_apart;
+    const bool apart = fuse && (ctx->fold_apart || blk);  // (a block's costs are folded apart)
     // a split level: chains [0, h) on st, [h, nchains) on st3 (h in whole workgroups)
     const int h = split_point(ctx);
-    const bool split = ctx->overlap && apart && h > 0 && h < ctx->nchains;
+    const bool split = ctx->overlap && apart && h > 0 && h < ctx->nchains && split_pays(ctx, blk);
     if (!split) TSA_HIP(ctx, join_split(ctx));
     // a resampling not yet made: this launch's kernel stages each chain from its ancestor's record (the chain
     // in LDS, one launch), else the copy first
@@ -1261,6 +1280,7 @@ extern "C" int tsa_track_begin(tsa_ctx* ctx, const tsa_select_t* sel, int32_t ma
   ctx->overlap = want_overlap;
   ctx->slot = 0;
   ctx->track_kind = 0;
+  ctx->anneal_blocks = false;
   ctx->lv_reset = true;
   ctx->lv_evaluated.assign((size_t)max_levels, 0);
   static_assert(sizeof(TsaTraceRowD) % 8 == 0, "trace rows are whole words");
@@ -1371,13 +1391,34 @@ static int track_wide_block(tsa_ctx* ctx, const int* slots, const int* levels, i
   return TSA_OK;
 }
 
+// Whether every chain of the level loop is resident on the device at once (an occupancy query of the one-wave
+// kernel, per mode and order).
+static int loop_fits(tsa_ctx* ctx, int32_t order, bool* fits) {
+  int& r = ctx->lv_resident[ctx->mode * 2 + order];
+  if (r < 0) {
+    TsaLevels q{};
+    TsaLaunch one = ctx->L;
+    one.team = one.team_float = 0;
+    const TsaEnergyOut eo{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    TSA_HIP(ctx, tsa_launch_sweeps(one, ctx->mode, order, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix, ctx->nchains,
+                                   0.0f, 0u, 0, ctx->d_stats, eo, ctx->st, nullptr, nullptr, &q, &r));
+  }
+  *fits = (long long)r * ctx->ncu >= ctx->nchains;
+  return TSA_OK;
+}
+
 extern "C" int tsa_track(tsa_ctx* ctx, int32_t level) {
   if (!ctx) return fail(ctx, TSA_ERR_ARG, "tsa_track: null context");
   if (ctx->track_levels == 0) return fail(ctx, TSA_ERR_ARG, "tsa_track: no tsa_track_begin");
   TSA_HIP(ctx, flush_track_init(ctx));
   TSA_HIP(ctx, flush_resample(ctx));
   if (level < 0 || level >= ctx->track_levels) return fail(ctx, TSA_ERR_ARG, "tsa_track: level out of range");
-  if (ctx->track_kind == TRACK_ANNEAL)
+  bool loop_session = ctx->track_kind == TRACK_ANNEAL;
+  if (!loop_session && ctx->anneal_blocks) {  // (a session whose levels tsa_anneal runs, whichever way it does)
+    const int rc = loop_fits(ctx, TSA_ORDER_PAR, &loop_session);
+    if (rc != TSA_OK) return rc;
+  }
+  if (loop_session)
     return fail(ctx, TSA_ERR_ARG, "tsa_track: this tracking session runs its levels with tsa_anneal");
   ctx->track_kind = TRACK_LEVELS;
   ctx->tend_staged = false;
@@ -1571,6 +1612,9 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
     nev += evaluated[l] != 0;
   }
   if (total > INT32_MAX) return fail(ctx, TSA_ERR_ARG, "tsa_anneal: more than 2^31 - 1 sweeps in one call");
+  if (ctx->cfg.level_blocks < 0 || ctx->cfg.level_blocks > TSA_BLOCK_MAX)
+    return fail(ctx, TSA_ERR_ARG, "tsa_config_t.level_blocks: 0 (automatic) or 1..8");
+  const int K = ctx->cfg.level_blocks > 0 ? ctx->cfg.level_blocks : TSA_BLOCK_MAX;
   // One launch for the whole call when the context's kernels run the level loop (the LDS kernels), it is not
   // turned off, and either it is asked for or every chain of it is resident at once: with more chains than
   // that, a chain resident only after others have run all their levels would leave the per-level launches'
@@ -1578,16 +1622,16 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
   // stays with it (the best is tracked per chain by the level loop, per level by tsa_track).
   bool loop = ctx->track_kind == TRACK_ANNEAL;
   if (ctx->track_kind == 0 && !ctx->wide.on && ctx->L.lds && ctx->cfg.level_loop >= 0) {
+    // ... or blocks of levels run instead: their folds of a level's energies run beside the next block's sweeps on
+    // lanes of their own, where the loop's chains fold serially between their levels (par order, 40 levels of one
+    // sweep: 72 chains of sat100 1.03 -> 0.55 ms, 768 1.41 -> 0.80, 3072 4.17 -> 1.88)
     loop = ctx->cfg.level_loop > 0;
     if (!loop) {
-      int& r = ctx->lv_resident[ctx->mode * 2 + order];
-      if (r < 0) {
-        TsaLevels q{};
-        const TsaEnergyOut eo{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-        TSA_HIP(ctx, tsa_launch_sweeps(ctx->L, ctx->mode, order, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix,
-                                       ctx->nchains, 0.0f, 0u, 0, ctx->d_stats, eo, ctx->st, nullptr, nullptr, &q, &r));
+      ctx->anneal_blocks = lds_blocks_ok(ctx, order, K);
+      if (!ctx->anneal_blocks) {
+        const int rc = loop_fits(ctx, order, &loop);
+        if (rc != TSA_OK) return rc;
       }
-      loop = (long long)r * ctx->ncu >= ctx->nchains;
     }
   }
   ctx->lv_used = loop ? 1 : 0;
@@ -1597,12 +1641,8 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
   // fewer and fewer chains are left to run, and a level of one sweep per chain is short next to it; a block of
   // levels has one tail for all of them.  Each evaluated level of a block leaves its snapshot in a slot of its
   // own, whose fold and selection tsa_track runs as for one level.
-  if (ctx->cfg.level_blocks < 0 || ctx->cfg.level_blocks > TSA_BLOCK_MAX)
-    return fail(ctx, TSA_ERR_ARG, "tsa_config_t.level_blocks: 0 (automatic) or 1..8");
-  const int K = ctx->cfg.level_blocks > 0 ? ctx->cfg.level_blocks : TSA_BLOCK_MAX;
   const bool wide_blocks = !loop && K > 1 && wide_blocks_ok(ctx, order);
-  if (wide_blocks || (!loop && K > 1 && ctx->overlap && !ctx->wide.on && ctx->L.lds && ctx->cfg.fused_energy != 0 &&
-                      ctx->fold_apart && !ctx->cfg.slicing && order == TSA_ORDER_PAR)) {
+  if (wide_blocks || (!loop && lds_blocks_ok(ctx, order, K))) {
     ctx->lv_used = 2;
     ctx->blocks_k = K;
     if (ensure_slots(ctx, 3 * K) != TSA_OK) return TSA_ERR_HIP;
@@ -1970,7 +2010,7 @@ extern "C" int tsa_sweeps_noalloc(const tsa_layout_t* lay, const tsa_config_t* c
   if (plan_one_wave(lay, cfg, nchains, d->lds_max, d->ncu, &L, &in_lds) != TSA_OK) return TSA_ERR_FIT;
   TsaKParams P;
   fill_params(*lay, *cfg, leaf_sc, P);
-  if (in_lds) L.team = tsa_team_plan(P, nchains, d->ncu, d->lds_max, cfg->wide_waves, &L.team_full);
+  if (in_lds) tsa_team_plan(P, nchains, d->ncu, d->lds_max, cfg->wide_waves, &L);
   hipStream_t st = static_cast<hipStream_t>(stream);
   unsigned long long* counters = reinterpret_cast<unsigned long long*>(d->scratch);
   float* cost = reinterpret_cast<float*>(d->scratch + kCounterBytes);

@@ -70,8 +70,9 @@ struct TsaLaunch {
   int lds_words;     // LDS words per wave
   int draw_waves;    // 1: pre-order sweeps run one chain per workgroup with helper waves that draw ahead
   int lds_max;       // dynamic LDS bytes a workgroup may have, less the kernel's static LDS
-  int team_full;     // k_team's long work-list entries
-  int team;          // par sweeps of a chain in LDS: waves per chain of k_team (0: k_sweep, one wave per chain)
+  // par sweeps of a chain in LDS: waves per chain of k_team in tc mode and in the float modes (0: k_sweep, one wave
+  // per chain), and whether its work-list entries are the long ones
+  int team, team_float, team_full;
 };
 
 // Helper waves per workgroup of a pre-order sweep with draws made ahead (the workgroup fills a compute unit's
@@ -201,9 +202,9 @@ hipError_t tsa_launch_team_sliced_compact(const TsaLaunch& L, int mode, const Ts
                                           const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
                                           unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
                                           hipEvent_t e1, const TsaLevels* lv, int* res);
-// Waves per chain for a par sweep of nchains chains with lds_max bytes of LDS per workgroup (0: k_sweep's one).  want:
-// 0 automatic, 1 one wave, 2..8 that many; *full: whether its work-list entries carry the node's words.
-int tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, int* full);
+// L's team fields for par sweeps of nchains chains with lds_max bytes of LDS per workgroup.  want: 0 automatic, 1 one
+// wave, 2..8 that many.
+void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, TsaLaunch* L);
 hipError_t tsa_launch_energy(int Wt, int mode, const TsaKParams& P, const uint64_t* rec, const uint64_t* leaf,
                              const uint32_t* fix, int nchains, float* lc, int* sc, int* ns, hipStream_t st);
 // The fold of node costs a sweep launch left in cost / z (nchains * nint4 each) into lc / sc / ns.

@@ -265,7 +265,7 @@ hipError_t tsa_launch_sweeps(const TsaLaunch& L, int mode, int order, const TsaK
                              hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res) {
   // (the team's visits take the costs before a move from a cache whose operands are in slot order, so its model may
   // not tell left from right: the gpu model does when m0 and n0 differ)
-  if (L.team > 0 && L.lds && order == 0 && eo.blk.n == 0 && (mode != 1 || P.model.m0 == P.model.n0)) {
+  if ((mode == 0 ? L.team : L.team_float) > 0 && L.lds && order == 0 && (mode != 1 || P.model.m0 == P.model.n0)) {
     const auto go = P.slicing ? (L.team_full ? tsa_launch_team_sliced_full : tsa_launch_team_sliced_compact)
                               : (L.team_full ? tsa_launch_team_full : tsa_launch_team_compact);
     return go(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);

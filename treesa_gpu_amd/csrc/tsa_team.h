@@ -304,9 +304,11 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
     s_cnt[0] = s_cnt[1] = 0;
     s_draw = 0;
   }
-  const int nsw = LVL ? Lv.total : nsweeps;
-  int lv = 0, left = LVL ? Lv.niters[0] : nsweeps;
-  float beta = LVL ? Lv.beta[0] : beta1;
+  // the level loop, a block of levels (eo.blk), or the launch's one level
+  const bool blocked = !LVL && eo.blk.n > 0;
+  const int nsw = LVL ? Lv.total : (blocked ? eo.blk.total : nsweeps);
+  int lv = 0, left = LVL ? Lv.niters[0] : (blocked ? eo.blk.niters[0] : nsweeps);
+  float beta = LVL ? Lv.beta[0] : (blocked ? eo.blk.beta[0] : beta1);
   for (int i = tid; i < nint; i += NT) draws[i] = tsa_team_draw(P, m + i, sweep0, (uint32_t)c);
   __syncthreads();
   if constexpr (MODE != 0) tsa_ilse_stage(s_ilse, T_);
@@ -603,6 +605,23 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
           left = F->Lv.niters[lv];
         }
       }
+    } else {
+      if (blocked && --left == 0) {  // a block's level ends: its snapshot (node costs, sizes, children words)
+        if (eo.blk.cost[lv]) {
+          float* const gc = eo.blk.cost[lv] + (size_t)c * nint4;
+          uint16_t* const gz = eo.blk.z[lv] + (size_t)c * nint4;
+          uint32_t* const gch = eo.blk.ch[lv] + (size_t)c * nint;
+          for (int i = tid; i < nint; i += NT) {
+            gc[i] = cc.cost(i);
+            gz[i] = (uint16_t)cc.size(i);
+            gch[i] = ch[i];
+          }
+        }
+        if (++lv < eo.blk.n) {
+          beta = eo.blk.beta[lv];
+          left = eo.blk.niters[lv];
+        }
+      }
     }
   }
   __syncthreads();
@@ -664,7 +683,7 @@ static hipError_t launch_team_t(const TsaLaunch& L, const TsaKParams& P, uint64_
                                 hipEvent_t e1, const TsaLevels* lv, int* res) {
   const int caches = tsa_team_caches(SLICE && P.slice_moves > 0, LVL);
   const size_t smem = (size_t)tsa_team_lds(P.m, P.nint, W, P.chain_words, MODE, caches, FULL).bytes;
-  const int threads = 64 * L.team;
+  const int threads = 64 * (MODE == 0 ? L.team : L.team_float);
   const void* const fn = reinterpret_cast<const void*>(&k_team<W, MODE, SLICE, LVL, FULL>);
   if (smem > 65536) {
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -672,6 +691,7 @@ static hipError_t launch_team_t(const TsaLaunch& L, const TsaKParams& P, uint64_
   }
   if (res) return hipOccupancyMaxActiveBlocksPerMultiprocessor(res, fn, threads, smem);  // a query, no launch
   if (P.chain0 < 0 || P.chain0 >= nchains) return hipErrorInvalidValue;
+  if (eo.blk.n > 0 && (LVL || eo.blk.n > TSA_BLOCK_MAX || eo.blk.total != nsweeps)) return hipErrorInvalidValue;
   hipExtLaunchKernelGGL((k_team<W, MODE, SLICE, LVL, FULL>), dim3(nchains - P.chain0), dim3(threads), (uint32_t)smem, st, e0,
                         e1, 0u, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, lv ? *lv : TsaLevels{});
   return hipGetLastError();
