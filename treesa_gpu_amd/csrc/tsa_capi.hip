@@ -72,6 +72,7 @@ struct tsa_ctx {
   // each chain's record from its ancestor's in d_rec and writes the population into d_rec2 (then the two swap);
   // any other call makes the copy first (flush_resample)
   bool anc_pend = false;
+  bool wide_pre = false;       // pre-order sweeps run tsa_wide_pre.hip (a wide context without slicing that fits)
   TsaWide wide{};              // wide path plan (wide.on: par sweeps and energies run tsa_wide.hip)
   TsaWideSync wsync{};         // chain barrier words (one allocation) and visit outcomes
   unsigned* d_wsync = nullptr;
@@ -531,16 +532,18 @@ extern "C" int tsa_create(const tsa_layout_t* lay, const uint64_t* leaf, int32_t
     // arithmetic of the lse chain, and adds a launch): worth it from three rounds of resident chains
     c->fold_apart = cfg->fused_energy == 2 || (long long)nchains > 2 * resident;
   }
-  // wide path: runtime-width chains without slice moves run par sweeps and energies in tsa_wide.hip
+  // wide path: runtime-width chains run par sweeps and energies in tsa_wide.hip
   const bool want_wide = cfg->kernel == TSA_KERNEL_WIDE || (cfg->kernel == TSA_KERNEL_AUTO && !use_lds);
   if (want_wide) {
     hipError_t we = hipErrorInvalidValue;
-    if (lay->runtime_width && !cfg->slicing)
+    // (slicing: on its own, with no plan asked for)
+    const bool asked = cfg->kernel == TSA_KERNEL_WIDE || cfg->wide_waves > 0 || cfg->wide_wgs > 0 || cfg->wide_lanes > 0;
+    if (lay->runtime_width && !(cfg->slicing && asked))
       we = tsa_wide_plan(c->P, nchains, cfg->wide_waves, cfg->wide_wgs, cfg->wide_lanes, cfg->sums, &c->wide);
     if (we != hipSuccess) {
       (void)hipGetLastError();  // clear the runtime's last error: the context goes on without the wide path
       c->wide = TsaWide{};
-      if (cfg->kernel == TSA_KERNEL_WIDE || cfg->wide_waves > 0 || cfg->wide_wgs > 0 || cfg->wide_lanes > 0) {
+      if (asked) {
         free_ctx(c);
         return fail(nullptr, TSA_ERR_FIT,
                     std::string("wide kernel: no plan (it needs runtime width, no slicing, W <= 256 words, lanes per "
@@ -550,6 +553,7 @@ extern "C" int tsa_create(const tsa_layout_t* lay, const uint64_t* leaf, int32_t
       }
     }
   }
+  c->wide_pre = c->wide.on && tsa_wide_pre_fits(c->P, lds_max);
   char kb[200];
   if (c->wide.on)
     snprintf(kb, sizeof kb,
@@ -929,12 +933,15 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
   if (blk && ctx->wide.on && !wide_blocks_ok(ctx, order))
     return fail(ctx, TSA_ERR_ARG, "block of levels on the wide path: one workgroup per chain, the overlapped "
                                   "selection with the fold apart, tc mode, par order");
-  if (ctx->wide.on && order == TSA_ORDER_PAR) {
+  const bool pre = order == TSA_ORDER_PREORDER;
+  if (ctx->wide.on && (!pre || ctx->wide_pre)) {
     TSA_HIP(ctx, join_split(ctx));
     TSA_HIP(ctx, flush_resample(ctx));
     // energies stay a separate fold of the node-cost cache: every chain ends its sweep at about the same
     // time, so folding inside the sweep kernel would only lengthen it
-    if (ctx->wide.nsw && !ctx->sums_valid) {
+    if (pre) {
+      ctx->sums_valid = false;  // (the pre-order kernel reads whole sets and keeps no summaries)
+    } else if (ctx->wide.nsw && !ctx->sums_valid) {
       TSA_HIP(ctx, tsa_launch_wsum(ctx->wide, ctx->P, ctx->d_rec, ctx->nchains, ctx->d_sum, ctx->st));
       ctx->sums_valid = true;
     }
@@ -942,7 +949,8 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
     int s = -1;
     // the node-cost cache must be exact before the sweep when the snapshot it leaves is folded as it stands,
     // and when the sweep reads it (tc mode: a visit takes P's old cost and size from it)
-    if ((ctx->overlap || ctx->mode == 0) && !ctx->costs_valid) {
+    // (a slicing sweep's moves fold it in every mode)
+    if ((ctx->overlap || ctx->mode == 0 || ctx->cfg.slicing) && !ctx->costs_valid) {
       join_track(ctx);
       TSA_HIP(ctx, tsa_launch_wide_energy(ctx->wide, ctx->mode, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix,
                                           ctx->nchains, ctx->d_ncost, ctx->d_nz, ctx->d_fcnt, ctx->d_lc, ctx->d_sc,
@@ -954,7 +962,8 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
     // group per chain): without the overlap into d_lc / d_sc / d_ns, with it into the snapshot slot, whose tree
     // the selection beside the next sweep reads
     const bool snap_fold = ctx->overlap && wide_fold_snap(ctx) && ctx->costs_valid;
-    const bool fold_here = !ctx->overlap && ctx->wide.K == 1 && ctx->wide.nsw == 0 && ctx->costs_valid;
+    const bool fold_here =
+        !ctx->overlap && (pre || (ctx->wide.K == 1 && ctx->wide.nsw == 0)) && ctx->costs_valid;
     if (fold_here) {
       join_track(ctx);  // a selection still pending on st2 reads d_lc / d_sc / d_ns
       sy.flc = ctx->d_lc;
@@ -994,8 +1003,12 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
       }
     }
     if (markers) TSA_HIP(ctx, hipEventRecord(e0, ctx->st));
-    TSA_HIP(ctx, tsa_launch_wide(ctx->wide, ctx->mode, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix, ctx->nchains, beta,
-                                 sweep0, nsweeps, ctx->d_stats, sy, ctx->st, d0, d1));
+    if (pre)
+      TSA_HIP(ctx, tsa_launch_wide_pre(ctx->mode, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix, ctx->nchains, ctx->ncu, beta,
+                                       sweep0, nsweeps, ctx->d_stats, sy, ctx->st, d0, d1));
+    else
+      TSA_HIP(ctx, tsa_launch_wide(ctx->wide, ctx->mode, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix, ctx->nchains, beta,
+                                   sweep0, nsweeps, ctx->d_stats, sy, ctx->st, d0, d1));
     if (markers) TSA_HIP(ctx, hipEventRecord(e1, ctx->st));
     if (s >= 0) {
       ctx->ev_sweep[s] = e1;  // the selection of this snapshot waits for the sweep's stop event
@@ -1269,7 +1282,7 @@ extern "C" int tsa_track_begin(tsa_ctx* ctx, const tsa_select_t* sel, int32_t ma
   // the records, so they keep the serial order.
   const bool want_overlap =
       ctx->cfg.track_overlap >= 0 &&
-      ((ctx->wide.on && ctx->wide.K == 1 && ctx->nchains < ctx->ncu) || wide_fold_snap(ctx) ||
+      ((ctx->wide.on && ctx->wide.K == 1 && ctx->nchains < ctx->ncu && !ctx->cfg.slicing) || wide_fold_snap(ctx) ||
        (!ctx->wide.on && ctx->cfg.fused_energy != 0 && !ctx->cfg.slicing));
   if (want_overlap && !ctx->st2) {
     TSA_HIP(ctx, hipStreamCreateWithFlags(&ctx->st2, hipStreamNonBlocking));

@@ -404,6 +404,9 @@ __host__ __device__ static inline TsaWideLds tsa_wide_lds(int nint, int band, in
   return L;
 }
 
+// LDS bytes a slicing launch of k_wide adds: two copies of the chain's node costs and sizes and of its slice set.
+__host__ __device__ static inline int tsa_wide_slice_bytes(int nint, int W) { return 2 * ((nint + 3) & ~3) * 6 + 2 * W * 8; }
+
 // Plan a wide launch for nchains chains on the current device: chunk summaries (sums: 1 on, -1 off, 0 on
 // from 64 words per set), lanes per proposal (want_g, 0 = from W, or 8 with summaries), threads per
 // workgroup (want_waves waves, 0 = by chain count), workgroups per chain (want_k, 0 = as many as stay
@@ -419,6 +422,13 @@ hipError_t tsa_launch_wide(const TsaWide& X, int mode, const TsaKParams& P, uint
                            const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
                            unsigned long long* stats, const TsaWideSync& sy, hipStream_t st,
                            hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+// Pre-order sweeps of wide chains without slicing (tsa_wide_pre.hip), the node-cost cache of X exact before (tc mode) and
+// kept; whether the context's chains fit it (lds_max: LDS bytes per workgroup).
+bool tsa_wide_pre_fits(const TsaKParams& P, int lds_max);
+hipError_t tsa_launch_wide_pre(int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf, const uint32_t* fix,
+                               int nchains, int ncu, float beta, uint32_t sweep0, int nsweeps,
+                               unsigned long long* stats, const TsaWideSync& sy, hipStream_t st,
+                               hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // Chunk summaries of the internal sets (isum[nchains][nint4][nsw]) and of the input tensors (lsum[m][nsw]) that
 // match the population; nsw = 0: none.
 struct TsaSums {

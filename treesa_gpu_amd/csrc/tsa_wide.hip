@@ -41,82 +41,9 @@
 // every workgroup that sees the error word stops, so every wave reaches the end of the kernel.  The last
 // workgroup of a chain to leave (all K of them leave, including those that only checked in) resets the
 // chain's words to zero for the next launch.
-#include "tsa_kernels.h"
-#include "tsa_fold.h"
+#include "tsa_wide.h"
 
 namespace {
-
-struct alignas(16) TsaW2 {
-  uint64_t a, b;
-};
-
-// Counters of one proposal as a flat list: |d|, |P|, |X|, then K0..K3 (mode 0) or B0..3, M0..3, N0..3,
-// K0..3 (modes 1, 2).
-template <int MODE>
-struct TsaFlat {
-  static constexpr int N = MODE == 0 ? 7 : 19;
-  static constexpr int NP = (N + 1) / 2;
-};
-
-template <int MODE>
-__device__ __forceinline__ void counts_pack(const TsaCounts& c, uint32_t (&a)[TsaFlat<MODE>::NP]) {
-  int f[TsaFlat<MODE>::NP * 2];
-  f[0] = c.sd;
-  f[1] = c.sp;
-  f[2] = c.sx;
-  if (MODE == 0) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) f[3 + q] = c.K[q];
-    f[7] = 0;
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      f[3 + q] = c.B[q];
-      f[7 + q] = c.M[q];
-      f[11 + q] = c.N[q];
-      f[15 + q] = c.K[q];
-    }
-    f[19] = 0;
-  }
-#pragma unroll
-  for (int i = 0; i < TsaFlat<MODE>::NP; i++) a[i] = (uint32_t)f[2 * i] | ((uint32_t)f[2 * i + 1] << 16);
-}
-
-template <int MODE>
-__device__ __forceinline__ void counts_unpack(const uint32_t (&a)[TsaFlat<MODE>::NP], TsaCounts& c) {
-  int f[TsaFlat<MODE>::NP * 2];
-#pragma unroll
-  for (int i = 0; i < TsaFlat<MODE>::NP; i++) {
-    f[2 * i] = (int)(a[i] & 0xFFFFu);
-    f[2 * i + 1] = (int)(a[i] >> 16);
-  }
-  c.sd = f[0];
-  c.sp = f[1];
-  c.sx = f[2];
-  if (MODE == 0) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) c.K[q] = f[3 + q];
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      c.B[q] = f[3 + q];
-      c.M[q] = f[7 + q];
-      c.N[q] = f[11 + q];
-      c.K[q] = f[15 + q];
-    }
-  }
-}
-
-// Sum over the G lanes of a group (xor butterfly: every lane ends with the total).  Each packed half
-// stays below 2^16: a label set has at most 2 * TSA_WIDE_CPL * 64 * 64 = 16384 labels.
-template <int G, int N>
-__device__ __forceinline__ void group_sum(uint32_t (&a)[N]) {
-#pragma unroll
-  for (int o = G / 2; o > 0; o >>= 1) {
-#pragma unroll
-    for (int i = 0; i < N; i++) a[i] += (uint32_t)__shfl_xor((int)a[i], o, G);
-  }
-}
 
 // Check-in of thread 0 (see the file comment): 0 sweep with the other K - 1, 1 sweep the chain alone, 2 leave.
 #define TSA_JOIN_CLAIMED 0x80000000u
@@ -178,11 +105,6 @@ __device__ bool chain_barrier(const TsaWideSync& sy, int c, unsigned target, int
   return *s_ok != 0;
 }
 
-__device__ __forceinline__ long long wide_wave_sum(long long x) {
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
-}
-
 // Chunk summaries: the chunks of a proposal are the set bits of the union u = u0 | u1 << 64 of the
 // summaries of D, O, K and M; lane t of a group of G takes the bits of rank t, t + G, t + 2G, ... so that the
 // loads spread evenly over the group whatever the positions, SC of them per round.  sum_pick returns the
@@ -211,54 +133,8 @@ __device__ __forceinline__ void sum_pick(uint64_t u0, uint64_t u1, int r, int (&
   }
 }
 
-// The fold of one chain's cached node costs by the calling workgroup: with stage >= 1 the costs (and with
-// stage 2 the log2f summary bitmap) are first copied into the workgroup's LDS at lds (vector copies, all
-// loads in flight at once: the fold reads them in a serial chain per lane); lanes 0..31 then fold in the
-// reference's order and lane 0 writes lc / sc / ns of chain c.  Every thread of the workgroup calls it.
-__device__ __forceinline__ void wide_fold(const TsaKParams& P, int c, const float* cst, const uint16_t* zz,
-                                          const uint64_t* S, const uint64_t* leaf, const uint32_t* fix,
-                                          const uint64_t* s_mt, int stage, unsigned char* lds, float* lc, int* sc,
-                                          int* ns) {
-  const int nint4 = (P.nint + 3) & ~3;
-  const uint32_t* const gmap = fix + TSA_LOG2FIX_WORDS;
-  const uint32_t* map = gmap;
-  if (stage) {
-    float* const scst = reinterpret_cast<float*>(lds);
-    uint16_t* const szz = reinterpret_cast<uint16_t*>(lds + (size_t)nint4 * 4);
-    const int n4 = nint4 / 4;
-#pragma unroll 4
-    for (int i = threadIdx.x; i < n4; i += blockDim.x) {
-      const float4 cv = reinterpret_cast<const float4*>(cst)[i];
-      const uint2 zv = reinterpret_cast<const uint2*>(zz)[i];
-      reinterpret_cast<float4*>(scst)[i] = cv;
-      reinterpret_cast<uint2*>(szz)[i] = zv;
-    }
-    if (stage == 2) {
-      uint4* const smap = reinterpret_cast<uint4*>(lds + (((size_t)nint4 * 6 + 15) & ~(size_t)15));
-      const uint4* src = reinterpret_cast<const uint4*>(gmap);
-#pragma unroll 16
-      for (int i = threadIdx.x; i < (int)(TSA_LOG2MAP_WORDS / 4); i += blockDim.x) smap[i] = src[i];
-      map = reinterpret_cast<const uint32_t*>(smap);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < 32) {
-    const TsaMathTabs T{s_mt, fix, map, s_mt + 32};
-    // two call sites, so that each inlined fold knows whether it reads LDS or global memory
-    const TsaEvalOut e = stage ? tsa_fold32(P, reinterpret_cast<const float*>(lds),
-                                            reinterpret_cast<const uint16_t*>(lds + (size_t)nint4 * 4), S, leaf, P.W,
-                                            T, (int)threadIdx.x)
-                               : tsa_fold32(P, cst, zz, S, leaf, P.W, T, (int)threadIdx.x);
-    if (threadIdx.x == 0) {
-      lc[c] = e.lcost;
-      sc[c] = e.sc;
-      ns[c] = e.ns;
-    }
-  }
-}
-
 // (SUMS: at most 512 threads, so that the summary visit has 256 registers and does not spill)
-template <int G, int MODE, bool COOP, bool SUMS>
+template <int G, int MODE, bool COOP, bool SUMS, bool SLICE>
 __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64_t* __restrict__ rec,
                                                const uint64_t* __restrict__ leaf, const uint32_t* __restrict__ fix,
                                                int nchains, int K, float beta0, uint32_t sweep0, int nsweeps,
@@ -267,6 +143,7 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
   __shared__ float s_lse[64];
   __shared__ uint64_t s_mt[TSA_MT_WORDS];
   __shared__ int s_cnt, s_ok, s_next, s_role;
+  __shared__ int s_move[2][2], s_acc;  // SLICE: proposed labels to add and remove (-1: none), two moves in turn
   const int NT = blockDim.x, nwv = NT >> 6, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = P.m, nint = P.nint, nint4 = (nint + 3) & ~3, ngrp = (nint + 63) >> 6;
   const int NW = P.W, nch = NW >> 1;
@@ -342,7 +219,34 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
   const int ngr = nwv * gpw;
   const int t = lane & (G - 1);
   const int gsub = lane / G;  // lane group within the wave
-  int np = 0, na = 0, nv = 0, nst = 0, nck = 0, nxk = 0;
+  int np = 0, na = 0, nv = 0, nst = 0, nck = 0, nxk = 0, nsp = 0, nsa = 0;
+  // the chain's node-cost cache: in HBM, or with SLICE in LDS for the launch (a second copy holds a proposed slice
+  // set's costs) with the slice set and the proposed one
+  float* cst = sy.ncost + (size_t)c * nint4;
+  uint16_t* cz = sy.nz + (size_t)c * nint4;
+  WideSlice sl{};
+  TsaW2 sm[SLICE ? tsa_wide_cpl(G) : 1];  // this lane's chunks of ~S
+  TsaEvalOut last_e{};
+  bool have_e = false;
+  auto load_mask = [&]() {
+    if constexpr (SLICE) {
+#pragma unroll
+      for (int q = 0; q < tsa_wide_cpl(G); q++) {
+        const int cc = t + q * G;
+        sm[q] = cc < nch ? TsaW2{~sl.S[2 * cc], ~sl.S[2 * cc + 1]} : TsaW2{0ull, 0ull};
+      }
+    }
+  };
+  if constexpr (SLICE) {
+    sl = wide_slice_lds(tsa_wsm + Lo.bytes, nint, NW);
+    tsa_copy_inflight<float, 4>(sl.cost, cst, nint, threadIdx.x, NT);
+    tsa_copy_inflight<uint16_t, 4>(sl.size, cz, nint, threadIdx.x, NT);
+    for (int i = threadIdx.x; i < NW; i += NT) sl.S[i] = lab[P.s_off + i];
+    cst = sl.cost;
+    cz = sl.size;
+    __syncthreads();
+    load_mask();
+  }
   unsigned nb = 0;
   bool ok = true;
   // a block of levels (one workgroup per chain, chunk summaries): the current level, its beta and its sweeps
@@ -488,6 +392,11 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
             const TsaW2* qO = reinterpret_cast<const TsaW2*>(On >= m ? lab + (size_t)(On - m) * NW : leaf + (size_t)On * NW);
             const TsaW2* qK = reinterpret_cast<const TsaW2*>(Kn >= m ? lab + (size_t)(Kn - m) * NW : leaf + (size_t)Kn * NW);
             const TsaW2* qM = reinterpret_cast<const TsaW2*>(Mn >= m ? lab + (size_t)(Mn - m) * NW : leaf + (size_t)Mn * NW);
+            bool acc;
+            if constexpr (!SUMS) {
+              acc = wide_visit_dense<G, MODE, SLICE>(P, T, s_lse, nch, t, Pn - m, v - m, slotP, slotM, qD, qP, qO, qK, qM,
+                                                     rnd.y, beta, cst, cz, sm);
+            } else {
             TsaCounts cn;
             tsa_counts_zero(cn);
             // tc mode: the costs of P and v before the move and P's size come from the node-cost cache
@@ -495,18 +404,16 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
             // P's set is never read
             int costP = 0, costV = 0, szP = 0;
             if constexpr (CACHED) {
-              const size_t cb = (size_t)c * nint4;
-              costP = (int)sy.ncost[cb + (Pn - m)];
-              costV = (int)sy.ncost[cb + (v - m)];
-              szP = (int)sy.nz[cb + (Pn - m)];
+              costP = (int)cst[Pn - m];
+              costV = (int)cst[v - m];
+              szP = (int)cz[Pn - m];
             }
             constexpr int SC = TsaSumRound<G>::SC;
-            constexpr int XN = SUMS ? SC : tsa_wide_cpl(G);
-            TsaW2 xx[XN];  // only X stays live across the energy evaluation
+            TsaW2 xx[SC];  // only X stays live across the energy evaluation
             // SUMS: the population count of the union (uniform in the group) and the chunk positions of this
             // lane's first round
             int pc = 0, ix[SC];
-            if constexpr (SUMS) {
+            {
               // summary word q of node n: LDS, or HBM for an input tensor whose table is not staged
               auto sumw = [&](int n, int q) -> uint64_t {
                 if (n >= m) return ssum[(size_t)(n - m) * nsw + q];
@@ -556,34 +463,6 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
                   }
                 }
               }
-            } else {
-              constexpr int CPL = tsa_wide_cpl(G);
-              TsaW2 dd[CPL], pp[CPL], oo[CPL], kk[CPL], mm[CPL];
-#pragma unroll
-              for (int q = 0; q < tsa_wide_cpl(G); q++) {
-                const int cc = t + q * G;
-                if (cc < nch) {
-                  dd[q] = qD[cc];
-                  if constexpr (!CACHED) pp[q] = qP[cc];
-                  oo[q] = qO[cc];
-                  kk[q] = qK[cc];
-                  mm[q] = qM[cc];
-                } else {
-                  dd[q] = pp[q] = oo[q] = kk[q] = mm[q] = TsaW2{0ull, 0ull};
-                }
-              }
-#pragma unroll
-              for (int q = 0; q < tsa_wide_cpl(G); q++) {
-                xx[q].a = tsa_xset(kk[q].a, oo[q].a, mm[q].a, dd[q].a);
-                xx[q].b = tsa_xset(kk[q].b, oo[q].b, mm[q].b, dd[q].b);
-                if constexpr (CACHED) {
-                  tsa_acc_after_tc(cn, kk[q].a, mm[q].a, oo[q].a, dd[q].a, xx[q].a);
-                  tsa_acc_after_tc(cn, kk[q].b, mm[q].b, oo[q].b, dd[q].b, xx[q].b);
-                } else {
-                  tsa_acc<MODE>(cn, kk[q].a, mm[q].a, pp[q].a, oo[q].a, dd[q].a, xx[q].a);
-                  tsa_acc<MODE>(cn, kk[q].b, mm[q].b, pp[q].b, oo[q].b, dd[q].b, xx[q].b);
-                }
-              }
             }
             float dE;
             if constexpr (CACHED) {
@@ -601,9 +480,9 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
               counts_unpack<MODE>(pk, cn);
               dE = tsa_energy_from_counts<MODE>(cn, P.model, s_lse, T);
             }
-            const bool acc = tsa_metropolis(rnd.y, beta, dE, T.exp2);
+            acc = tsa_metropolis(rnd.y, beta, dE, T.exp2);
             if (acc) {
-              if constexpr (SUMS) {
+              {
                 // X's chunks inside the union, and P's new summary (OR over the group).  The first round's
                 // chunks are still in registers; later rounds (more than SC * G chunks, rare) rebuild the union
                 // and the set pointers from LDS, so that neither stays live across the energy evaluation
@@ -669,32 +548,18 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
                     gsum[(size_t)(Pn - m) * nsw + 1] = xs1;
                   }
                 }
-              } else {
-#pragma unroll
-                for (int q = 0; q < tsa_wide_cpl(G); q++) {
-                  const int cc = t + q * G;
-                  if (cc < nch) qP[cc] = xx[q];
-                }
               }
+              if (t == 0) wide_cache_accept<MODE>(P, T, cn, Pn - m, v - m, slotP, slotM, cst, cz);
             }
-            if (SUMS && t == 0) {
+            if (t == 0) {
               nck += pc;
               nxk += acc ? pc : 0;
+            }
             }
             o = 8u | (acc ? 1u : 0u) | ((uint32_t)slotP << 1) | ((uint32_t)slotM << 2);
             if (t == 0) {
               np++;
               na += acc ? 1 : 0;
-              if (acc) {
-                // the two node costs the rotation changes: P with children K and O (O in M's slot) and v with
-                // children P and M (M in O's slot); count3 order is (left child, right child, node)
-                const size_t cb = (size_t)c * nint4;
-                sy.ncost[cb + (Pn - m)] = tsa_node_cost<MODE>(cn.B[2], slotM ? cn.M[2] : cn.N[2],
-                                                              slotM ? cn.N[2] : cn.M[2], cn.K[2], cn.sx, P.model, T);
-                sy.nz[cb + (Pn - m)] = (uint16_t)cn.sx;
-                sy.ncost[cb + (v - m)] = tsa_node_cost<MODE>(cn.B[3], slotP ? cn.N[3] : cn.M[3],
-                                                             slotP ? cn.M[3] : cn.N[3], cn.K[3], cn.sd, P.model, T);
-              }
             }
           }
           if (t == 0) {
@@ -743,6 +608,16 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
       }
       __syncthreads();
     }
+    if constexpr (SLICE) {
+      have_e = false;
+      if (P.slice_moves > 0 && (sw + 1u) % (uint32_t)P.slice_every == 0u) {
+        __syncthreads();
+        have_e = wide_slice_step<MODE>(P, lab, ch, sl, leaf, T, beta, sw, (uint32_t)c, s_move, &s_acc, nsp, nsa, last_e);
+        cst = sl.cost;
+        cz = sl.size;
+        load_mask();
+      }
+    }
     if (blocked && --left == 0) {
       // the level's end: its snapshot, the tree from LDS and the node-cost cache (final after the sweep's last
       // barrier), read by all before the next level's first accept rewrites the cache
@@ -761,6 +636,15 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
     }
   }
 
+  if constexpr (SLICE) {  // the cache and the slice set back to HBM
+    float* const gcst = sy.ncost + (size_t)c * nint4;
+    uint16_t* const gz = sy.nz + (size_t)c * nint4;
+    for (int i = threadIdx.x; i < nint; i += NT) {
+      gcst[i] = cst[i];
+      gz[i] = cz[i];
+    }
+    for (int i = threadIdx.x; i < NW; i += NT) lab[P.s_off + i] = sl.S[i];
+  }
   if (ok && ke == 0) {
     for (int i = threadIdx.x; i < nint; i += NT) gch[i] = ch[i];
     if (sy.snap_ch) {  // the level's snapshot: tree from LDS, node costs (final after the last barrier)
@@ -777,7 +661,13 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
     // the launch's energies, folded by this workgroup rather than by a launch of their own: every accept
     // rewrote its entries of the node-cost cache before the loop's last barrier, so the cache is the final
     // tree's; the costs are staged in the sweep's LDS, whose last reads (the tree, above) end at the barrier
-    if (sy.flc) {
+    if (SLICE && sy.flc && have_e) {  // the last slice step folded the chain as it stands
+      if (threadIdx.x == 0) {
+        sy.flc[c] = last_e.lcost;
+        sy.fsc[c] = last_e.sc;
+        sy.fns[c] = last_e.ns;
+      }
+    } else if (sy.flc) {
       __syncthreads();
       const size_t cb = (size_t)c * nint4;
       wide_fold(P, c, sy.ncost + cb, sy.nz + cb, P.slicing ? lab + P.s_off : nullptr, leaf, fix, s_mt,
@@ -793,6 +683,10 @@ __global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64
     atomicAdd(&st[TSA_ST_VISITS * TSA_STAT_SLOTS], (unsigned long long)sv_);
     atomicAdd(&st[TSA_ST_BUSY * TSA_STAT_SLOTS], (unsigned long long)sv_);
     if (ke == 0 && wv == 0) atomicAdd(&st[TSA_ST_STEPS * TSA_STAT_SLOTS], (unsigned long long)nst);
+    if (SLICE && wv == 0) {
+      atomicAdd(&st[TSA_ST_SPROP * TSA_STAT_SLOTS], (unsigned long long)nsp);
+      atomicAdd(&st[TSA_ST_SACC * TSA_STAT_SLOTS], (unsigned long long)nsa);
+    }
     if (SUMS) {
       atomicAdd(&st[TSA_ST_CHUNKS * TSA_STAT_SLOTS], (unsigned long long)sk_);
       atomicAdd(&st[TSA_ST_XCHUNKS * TSA_STAT_SLOTS], (unsigned long long)sx_);
@@ -935,16 +829,26 @@ hipError_t launch_wide_gms(const TsaWide& X, const TsaKParams& P, uint64_t* rec,
                            hipEvent_t e1) {
   // e0 / e1 (null: none) take the kernel's start and stop times in the dispatch itself
   if (X.K > 1) {
+    if (P.slicing) return hipErrorInvalidValue;
     // an ordinary launch: the plan admits K > 1 only when all nchains * K workgroups fit on the device at
     // once, so on an idle device they are all resident together (the cooperative launch API gives the same
     // guarantee but costs tens of microseconds per launch on the host side); if they ever are not, a chain
     // barrier runs out of polls, sets the error word and every workgroup leaves
     const int nchainsx = (nchains + X.nxcd - 1) / X.nxcd * X.nxcd;  // (chains grouped by XCD, see k_wide)
-    hipExtLaunchKernelGGL((k_wide<G, MODE, true, SUMS>), dim3(nchainsx * X.K), dim3(X.nt), (uint32_t)X.smem, st, e0,
+    hipExtLaunchKernelGGL((k_wide<G, MODE, true, SUMS, false>), dim3(nchainsx * X.K), dim3(X.nt), (uint32_t)X.smem, st, e0,
                           e1, 0u, P, rec, leaf, fix, nchains, X.K, beta, sweep0, nsweeps, stats, sy);
     return hipGetLastError();
   }
-  hipExtLaunchKernelGGL((k_wide<G, MODE, false, SUMS>), dim3(nchains), dim3(X.nt), (uint32_t)X.smem, st, e0, e1, 0u,
+  if constexpr (!SUMS) {
+    if (P.slicing) {
+      const int smem = X.smem + tsa_wide_slice_bytes(P.nint, P.W);
+      hipExtLaunchKernelGGL((k_wide<G, MODE, false, false, true>), dim3(nchains), dim3(X.nt), (uint32_t)smem, st, e0, e1, 0u,
+                            P, rec, leaf, fix, nchains, 1, beta, sweep0, nsweeps, stats, sy);
+      return hipGetLastError();
+    }
+  }
+  if (P.slicing) return hipErrorInvalidValue;  // (the plan of a slicing context is dense, one workgroup per chain)
+  hipExtLaunchKernelGGL((k_wide<G, MODE, false, SUMS, false>), dim3(nchains), dim3(X.nt), (uint32_t)X.smem, st, e0, e1, 0u,
                         P, rec, leaf, fix, nchains, 1, beta, sweep0, nsweeps, stats, sy);
   return hipGetLastError();
 }
@@ -997,15 +901,22 @@ hipError_t launch_wcost_g(const TsaWide& X, int mode, const TsaKParams& P, const
 // lds_cap first (the largest any context asks for).
 template <int G, bool SUMS>
 hipError_t wide_occupancy(int nt, int smem, int lds_cap, int* per_cu) {
-  const void* coop[3] = {reinterpret_cast<const void*>(&k_wide<G, 0, true, SUMS>),
-                         reinterpret_cast<const void*>(&k_wide<G, 1, true, SUMS>),
-                         reinterpret_cast<const void*>(&k_wide<G, 2, true, SUMS>)};
-  const void* one[3] = {reinterpret_cast<const void*>(&k_wide<G, 0, false, SUMS>),
-                        reinterpret_cast<const void*>(&k_wide<G, 1, false, SUMS>),
-                        reinterpret_cast<const void*>(&k_wide<G, 2, false, SUMS>)};
-  for (int i = 0; i < 6; i++) {
-    const hipError_t e =
-        hipFuncSetAttribute(i < 3 ? coop[i] : one[i - 3], hipFuncAttributeMaxDynamicSharedMemorySize, lds_cap);
+  const void* coop[3] = {reinterpret_cast<const void*>(&k_wide<G, 0, true, SUMS, false>),
+                         reinterpret_cast<const void*>(&k_wide<G, 1, true, SUMS, false>),
+                         reinterpret_cast<const void*>(&k_wide<G, 2, true, SUMS, false>)};
+  const void* one[3] = {reinterpret_cast<const void*>(&k_wide<G, 0, false, SUMS, false>),
+                        reinterpret_cast<const void*>(&k_wide<G, 1, false, SUMS, false>),
+                        reinterpret_cast<const void*>(&k_wide<G, 2, false, SUMS, false>)};
+  const void* sliced[3] = {nullptr, nullptr, nullptr};
+  if constexpr (!SUMS) {
+    sliced[0] = reinterpret_cast<const void*>(&k_wide<G, 0, false, false, true>);
+    sliced[1] = reinterpret_cast<const void*>(&k_wide<G, 1, false, false, true>);
+    sliced[2] = reinterpret_cast<const void*>(&k_wide<G, 2, false, false, true>);
+  }
+  for (int i = 0; i < 9; i++) {
+    const void* const f = i < 3 ? coop[i] : i < 6 ? one[i - 3] : sliced[i - 6];
+    if (!f) continue;
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_cap);
     if (e != hipSuccess) return e;
   }
   int best = 1 << 30;
@@ -1094,7 +1005,8 @@ hipError_t tsa_wide_plan(const TsaKParams& P, int nchains, int want_waves, int w
   // dense streaming needs G * tsa_wide_cpl(G) >= chunks per set; the energy kernel always streams densely
   int Gd = 4;
   while (Gd < 64 && (nch + Gd - 1) / Gd > tsa_wide_cpl(Gd)) Gd *= 2;
-  X.nsw = (sums > 0 || (sums == 0 && P.W >= 64)) ? (nch + 63) / 64 : 0;
+  // (slicing: dense, one workgroup per chain)
+  X.nsw = !P.slicing && (sums > 0 || (sums == 0 && P.W >= 64)) ? (nch + 63) / 64 : 0;
   // summaries: one lane per proposal (the union of a visit is a few chunks: whole-wave SIMD efficiency
   // matters more than spreading loads) and one workgroup per chain (no chain barriers)
   int G = want_g > 0 ? want_g : (X.nsw ? 1 : Gd);
@@ -1135,7 +1047,7 @@ hipError_t tsa_wide_plan(const TsaKParams& P, int nchains, int want_waves, int w
   }
   const int mlds = X.lsum_lds ? P.m : 0;
   const TsaWideLds L1 = tsa_wide_lds(P.nint, band, 0, X.nsw, mlds), Lc = tsa_wide_lds(P.nint, band, 1, X.nsw, mlds);
-  if (L1.bytes > lds_cap) return hipErrorInvalidValue;
+  if (L1.bytes + (P.slicing ? tsa_wide_slice_bytes(P.nint, P.W) : 0) > lds_cap) return hipErrorInvalidValue;
   // the fold stages a chain's node costs (6 B per node) and, when it also fits, the log2f summary bitmap
   X.fold_smem = nint4 * 6 <= lds_cap ? nint4 * 6 : 0;
   X.fold_smem_map = ((nint4 * 6 + 15) & ~15) + (int)TSA_LOG2MAP_WORDS * 4;
@@ -1149,7 +1061,7 @@ hipError_t tsa_wide_plan(const TsaKParams& P, int nchains, int want_waves, int w
   // be resident on its ncu / nxcd compute units at once (when they are not -- the device is shared with other
   // work -- a chain's check-in times out and one of its workgroups sweeps it alone)
   const int kmax = per_cu * (ncu / nxcd) / ((nchains + nxcd - 1) / nxcd);
-  int K = want_k > 0 ? want_k : (X.nsw ? 1 : kmax);
+  int K = want_k > 0 ? want_k : (X.nsw || P.slicing ? 1 : kmax);
   K = K < 1 ? 1 : (K > TSA_WIDE_MAX_K ? TSA_WIDE_MAX_K : K);
   if (K > 1 && K > kmax) return hipErrorCooperativeLaunchTooLarge;
   X.K = K;
