@@ -133,9 +133,9 @@ __device__ __forceinline__ void sum_pick(uint64_t u0, uint64_t u1, int r, int (&
   }
 }
 
-// (SUMS: at most 512 threads, so that the summary visit has 256 registers and does not spill)
+// (SUMS, SLICE: at most 512 threads, so that the visit and the slice step have 256 registers and do not spill)
 template <int G, int MODE, bool COOP, bool SUMS, bool SLICE>
-__global__ void __launch_bounds__(SUMS ? 512 : 1024) k_wide(TsaKParams P, uint64_t* __restrict__ rec,
+__global__ void __launch_bounds__(SUMS || SLICE ? 512 : 1024) k_wide(TsaKParams P, uint64_t* __restrict__ rec,
                                                const uint64_t* __restrict__ leaf, const uint32_t* __restrict__ fix,
                                                int nchains, int K, float beta0, uint32_t sweep0, int nsweeps,
                                                unsigned long long* __restrict__ stats, TsaWideSync sy) {
@@ -1023,10 +1023,12 @@ hipError_t tsa_wide_plan(const TsaKParams& P, int nchains, int want_waves, int w
     nxcd = 1;
   }
   X.nxcd = nxcd;
+  // (slicing: 8 waves at 256 registers, where 16 at 128 spill a hundred: 24 x 24 lattice, 128 chains, 66 against 79 us a
+  // sweep)
   // measured on MI355X: with at least one chain per CU, one 8-wave workgroup per chain streams best; with
   // fewer chains, 16-wave workgroups, as many per chain as stay co-resident
   // (the summary path is compiled for at most 8 waves per workgroup: its visit needs more registers)
-  const int max_waves = X.nsw ? 8 : 16;
+  const int max_waves = X.nsw || P.slicing ? 8 : 16;
   int waves = want_waves > 0 ? want_waves : (nchains >= ncu ? 8 : max_waves);
   waves = waves < 1 ? 1 : (waves > max_waves ? max_waves : waves);
   X.nt = 64 * waves;
