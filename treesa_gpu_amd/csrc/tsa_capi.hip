@@ -1411,7 +1411,7 @@ static int loop_fits(tsa_ctx* ctx, int32_t order, bool* fits) {
   if (r < 0) {
     TsaLevels q{};
     TsaLaunch one = ctx->L;
-    one.team = one.team_float = 0;
+    one.team = one.team_float = one.team_pre = 0;
     const TsaEnergyOut eo{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     TSA_HIP(ctx, tsa_launch_sweeps(one, ctx->mode, order, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix, ctx->nchains,
                                    0.0f, 0u, 0, ctx->d_stats, eo, ctx->st, nullptr, nullptr, &q, &r));

@@ -73,6 +73,7 @@ struct TsaLaunch {
   // par sweeps of a chain in LDS: waves per chain of k_team in tc mode and in the float modes (0: k_sweep, one wave
   // per chain), and whether its work-list entries are the long ones
   int team, team_float, team_full;
+  int team_pre;      // pre-order sweeps with helper waves (draw_waves) run k_team_pre
 };
 
 // Helper waves per workgroup of a pre-order sweep with draws made ahead (the workgroup fills a compute unit's
@@ -202,6 +203,13 @@ hipError_t tsa_launch_team_sliced_compact(const TsaLaunch& L, int mode, const Ts
                                           const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
                                           unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
                                           hipEvent_t e1, const TsaLevels* lv, int* res);
+// Pre-order sweeps of chains in LDS with helper waves, without slicing (tsa_team_pre.hip); res as above.  Whether a chain
+// fits (lds_max: LDS bytes per workgroup).
+bool tsa_team_pre_fits(const TsaKParams& P, int lds_max);
+hipError_t tsa_launch_team_pre(int W, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
+                               const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
+                               unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
+                               hipEvent_t e1, const TsaLevels* lv, int* res);
 // L's team fields for par sweeps of nchains chains with lds_max bytes of LDS per workgroup.  want: 0 automatic, 1 one
 // wave, 2..8 that many.
 void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, TsaLaunch* L);

@@ -270,6 +270,8 @@ hipError_t tsa_launch_sweeps(const TsaLaunch& L, int mode, int order, const TsaK
                               : (L.team_full ? tsa_launch_team_full : tsa_launch_team_compact);
     return go(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
   }
+  if (L.team_pre && L.lds && L.draw_waves && order == 1 && !P.slicing && (mode != 1 || P.model.m0 == P.model.n0))
+    return tsa_launch_team_pre(L.W, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
   if (P.slicing)
     return tsa_launch_sweeps_sliced(L, mode, order, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st,
                                     e0, e1, lv, res);

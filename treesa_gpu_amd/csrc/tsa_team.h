@@ -115,6 +115,122 @@ __device__ __forceinline__ uint32_t tsa_team_draw(const TsaKParams& P, int v, ui
   return (r.y & 0xFFFFFF00u) | (r.x >> 30);
 }
 
+// A visit's outcome: the children words of v and of the pivot after it, the pivot's cost word, the nodes it moved.
+struct TsaTeamMove {
+  uint32_t chv, chp, cp;
+  int Pn, On, Mn;
+  bool acc;
+};
+__device__ __forceinline__ bool tsa_team_has_rule(uint32_t chv, int m) {
+  return (int)(chv & 0xFFFFu) >= m || (int)(chv >> 16) >= m;
+}
+// One proposal at the node of work-list entry w (children word, draw, cost word, id; it has a rule), by a group of G lanes
+// (this one t): dE from the counts after the move and the cached costs before it, the Metropolis test, and when accepted
+// the pivot's new set, the two children words and the cache (leader lane).  early(On, Mn): called once both are known,
+// before the label sets arrive, for reads a caller wants in flight beside them.
+template <int W, int MODE, bool SLICE, class Early>
+__device__ __forceinline__ TsaTeamMove tsa_team_visit(const TsaKParams& P, uint64_t* lab, uint32_t* ch,
+                                                      const TsaTeamCache<MODE>& cc, const uint64_t* S,
+                                                      const float* s_lse, const float* s_ilse, const TsaMathTabs& T,
+                                                      const uint4& w, float beta, int t, Early early) {
+  constexpr int G = TsaTeamShape<W, MODE>::G, WL = TsaTeamShape<W, MODE>::WL, NC = MODE == 0 ? 4 : 10;
+  const int m = P.m, vi = (int)w.w - m;
+  const uint32_t chv = w.x, d = w.y;
+  const int l = (int)(chv & 0xFFFFu), r = (int)(chv >> 16);
+  const bool li = l >= m, ri = r >= m;
+  const float costV = MODE == 0 ? (float)(w.z & 0xFFFFu) : __uint_as_float(w.z);
+  const int b2 = (int)(d & 3u);
+  const int rule = li && ri ? b2 : (li ? b2 >> 1 : 2 + (b2 >> 1));
+  const int slotP = tsa_slot_p(rule), slotM = tsa_slot_m(rule);
+  const int Pn = slotP ? r : l, On = slotP ? l : r, pi = Pn - m;
+  const uint32_t chp = ch[pi], cp = cc.a[pi];
+  const float costP = MODE == 0 ? (float)(cp & 0xFFFFu) : __uint_as_float(cp);
+  const int szP = MODE == 0 ? (int)(cp >> 16) : (int)cc.z[pi];
+  const int Mn = slotM ? (int)(chp >> 16) : (int)(chp & 0xFFFFu);
+  const int Kn = slotM ? (int)(chp & 0xFFFFu) : (int)(chp >> 16);
+  const int w0 = t * WL;
+  const bool has = W >= G || t < W;  // (the float modes' second lane of a one-word set has none)
+  uint64_t xd[WL], xo[WL], xk[WL], xm[WL], xx[WL];
+  int pk[NC];
+#pragma unroll
+  for (int q = 0; q < NC; q++) pk[q] = 0;
+  if (has) {
+    tsa_load_words<WL>(lab + vi * W + w0, xd);
+    tsa_load_words<WL>(lab + (On - m) * W + w0, xo);
+    tsa_load_words<WL>(lab + (Kn - m) * W + w0, xk);
+    tsa_load_words<WL>(lab + (Mn - m) * W + w0, xm);
+  }
+  early(On, Mn);
+  if (has) {
+#pragma unroll
+    for (int i = 0; i < WL; i++) {
+      xx[i] = tsa_xset(xk[i], xo[i], xm[i], xd[i]);
+      uint64_t k = xk[i], o = xo[i], mm = xm[i], dd = xd[i], x = xx[i];
+      if constexpr (SLICE) {
+        const uint64_t nm = ~S[w0 + i];
+        k &= nm;
+        o &= nm;
+        mm &= nm;
+        dd &= nm;
+        x &= nm;
+      }
+      pk[0] += tsa_popc64(dd);
+      pk[1] += tsa_popc64(x);
+      if constexpr (MODE == 0) {
+        pk[2] += tsa_popc3<TSA_F_AB_NC>(k, o, x);
+        pk[3] += tsa_popc3<TSA_F_AB_NC>(x, mm, dd);
+      } else {
+        tsa_count3(k, o, x, pk[2], pk[3], pk[4], pk[5]);
+        tsa_count3(x, mm, dd, pk[6], pk[7], pk[8], pk[9]);
+      }
+    }
+  }
+  if constexpr (G > 1) {
+#pragma unroll
+    for (int q = 0; q < NC; q += 2) {
+      const uint32_t z = tsa_group_sum<G>((uint32_t)pk[q] | ((uint32_t)pk[q + 1] << 16));
+      pk[q] = (int)(z & 0xFFFFu);
+      pk[q + 1] = (int)(z >> 16);
+    }
+  }
+  const int sd = pk[0], sx = pk[1];
+  float dE, newP, newV;
+  if constexpr (MODE == 0) {
+    dE = tsa_energy_tc_cached((int)costP, (int)costV, szP, sd, sx, pk[2], pk[3], P.model, s_lse);
+    newP = (float)(sx + pk[2]);
+    newV = (float)(sd + pk[3]);
+  } else {
+    // even lanes cost the new P = (K, O), odd lanes the new v = (P, M); then the even lanes fold the pair after the move
+    // while the odd ones fold the pair before it
+    const int q = t & 1;
+    const float mine = tsa_node_cost_i<MODE>(q ? pk[6] : pk[2], q ? pk[7] : pk[3], q ? pk[8] : pk[4], q ? pk[9] : pk[5],
+                                             P.model, T, s_ilse);
+    const float other = __uint_as_float(tsa_dpp_xor1(__float_as_uint(mine)));
+    newP = q ? other : mine;
+    newV = q ? mine : other;
+    const float h = tsa_lse_f(q ? costP : newP, q ? costV : newV, T);
+    const float ho = __uint_as_float(tsa_dpp_xor1(__float_as_uint(h)));
+    const float dtc = q ? ho - h : h - ho;
+    const int sc0 = szP > sd ? szP : sd, sc1 = sx > sd ? sx : sd, scm = sc0 > sc1 ? sc0 : sc1;
+    const float pw = ((float)scm > P.model.sc_target) ? P.model.sc_weight : 0.0f;
+    dE = pw * (float)(sc1 - sc0) + dtc;
+  }
+  TsaTeamMove o{chv, chp, cp, Pn, On, Mn, tsa_metropolis(d, beta, dE, T.exp2)};
+  if (o.acc) {
+    if (has) tsa_store_words<WL>(lab + pi * W + w0, xx);
+    o.chp = slotM ? ((chp & 0xFFFFu) | ((uint32_t)On << 16)) : ((chp & 0xFFFF0000u) | (uint32_t)On);
+    o.chv = slotP ? ((chv & 0xFFFF0000u) | (uint32_t)Mn) : ((chv & 0xFFFFu) | ((uint32_t)Mn << 16));
+    o.cp = MODE == 0 ? ((uint32_t)newP | ((uint32_t)sx << 16)) : __float_as_uint(newP);
+    if (t == 0) {
+      ch[pi] = o.chp;
+      ch[vi] = o.chv;
+      cc.set(pi, newP, sx);
+      cc.set(vi, newV, sd);
+    }
+  }
+  return o;
+}
+
 // 64-node groups of a wave's scan batch; rows of a pending level fold per phase (7 phases or so cover a tree of a few
 // hundred nodes, so that the tracking wave's fold hides behind the phases of the next sweep).
 #define TSA_TEAM_SCAN 2
@@ -469,99 +585,13 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
           w = wl4[j];
         }
         const int v = (int)w.w, vi = v - m;
-        const uint32_t chv = w.x, d = w.y;
-        const int l = (int)(chv & 0xFFFFu), r = (int)(chv >> 16);
-        const bool li = l >= m, ri = r >= m;
-        if (li || ri) {
-          const float costV = MODE == 0 ? (float)(w.z & 0xFFFFu) : __uint_as_float(w.z);
-          const int b2 = (int)(d & 3u);
-          const int rule = li && ri ? b2 : (li ? b2 >> 1 : 2 + (b2 >> 1));
-          const int slotP = tsa_slot_p(rule), slotM = tsa_slot_m(rule);
-          const int Pn = slotP ? r : l, On = slotP ? l : r, pi = Pn - m;
-          const uint32_t chp = ch[pi];
-          const float costP = cc.cost(pi);
-          const int szP = cc.size(pi);
-          const int Mn = slotM ? (int)(chp >> 16) : (int)(chp & 0xFFFFu);
-          const int Kn = slotM ? (int)(chp & 0xFFFFu) : (int)(chp >> 16);
-          const int w0 = t * WL;
-          const bool has = W >= G || t < W;  // (the float modes' second lane of a one-word set has none)
-          uint64_t xd[WL], xo[WL], xk[WL], xm[WL], xx[WL];
-          int pk[MODE == 0 ? 4 : 10];
-#pragma unroll
-          for (int q = 0; q < (MODE == 0 ? 4 : 10); q++) pk[q] = 0;
-          if (has) {
-            tsa_load_words<WL>(lab + vi * W + w0, xd);
-            tsa_load_words<WL>(lab + (On - m) * W + w0, xo);
-            tsa_load_words<WL>(lab + (Kn - m) * W + w0, xk);
-            tsa_load_words<WL>(lab + (Mn - m) * W + w0, xm);
-#pragma unroll
-            for (int i = 0; i < WL; i++) {
-              xx[i] = tsa_xset(xk[i], xo[i], xm[i], xd[i]);
-              uint64_t k = xk[i], o = xo[i], mm = xm[i], dd = xd[i], x = xx[i];
-              if constexpr (SLICE) {
-                const uint64_t nm = ~S[w0 + i];
-                k &= nm;
-                o &= nm;
-                mm &= nm;
-                dd &= nm;
-                x &= nm;
-              }
-              pk[0] += tsa_popc64(dd);
-              pk[1] += tsa_popc64(x);
-              if constexpr (MODE == 0) {
-                pk[2] += tsa_popc3<TSA_F_AB_NC>(k, o, x);
-                pk[3] += tsa_popc3<TSA_F_AB_NC>(x, mm, dd);
-              } else {
-                tsa_count3(k, o, x, pk[2], pk[3], pk[4], pk[5]);
-                tsa_count3(x, mm, dd, pk[6], pk[7], pk[8], pk[9]);
-              }
-            }
-          }
-          if constexpr (G > 1) {
-#pragma unroll
-            for (int q = 0; q < (MODE == 0 ? 4 : 10); q += 2) {
-              const uint32_t z = tsa_group_sum<G>((uint32_t)pk[q] | ((uint32_t)pk[q + 1] << 16));
-              pk[q] = (int)(z & 0xFFFFu);
-              pk[q + 1] = (int)(z >> 16);
-            }
-          }
-          const int sd = pk[0], sx = pk[1];
-          float dE, newP, newV;
-          if constexpr (MODE == 0) {
-            dE = tsa_energy_tc_cached((int)costP, (int)costV, szP, sd, sx, pk[2], pk[3], P.model, s_lse);
-            newP = (float)(sx + pk[2]);
-            newV = (float)(sd + pk[3]);
-          } else {
-            // even lanes cost the new P = (K, O), odd lanes the new v = (P, M); then the even lanes fold the pair
-            // after the move while the odd ones fold the pair before it
-            const int q = t & 1;
-            const float mine = tsa_node_cost_i<MODE>(q ? pk[6] : pk[2], q ? pk[7] : pk[3], q ? pk[8] : pk[4],
-                                                     q ? pk[9] : pk[5], P.model, T_, s_ilse);
-            const float other = __uint_as_float(tsa_dpp_xor1(__float_as_uint(mine)));
-            newP = q ? other : mine;
-            newV = q ? mine : other;
-            const float h = tsa_lse_f(q ? costP : newP, q ? costV : newV, T_);
-            const float ho = __uint_as_float(tsa_dpp_xor1(__float_as_uint(h)));
-            const float dtc = q ? ho - h : h - ho;
-            const int sc0 = szP > sd ? szP : sd, sc1 = sx > sd ? sx : sd, scm = sc0 > sc1 ? sc0 : sc1;
-            const float w = ((float)scm > P.model.sc_target) ? P.model.sc_weight : 0.0f;
-            dE = w * (float)(sc1 - sc0) + dtc;
-          }
-          const bool acc = tsa_metropolis(d, beta, dE, s_mt);
-          if (acc) {
-            if (has) tsa_store_words<WL>(lab + pi * W + w0, xx);
-            if (t == 0) {
-              ch[pi] = slotM ? ((chp & 0xFFFFu) | ((uint32_t)On << 16)) : ((chp & 0xFFFF0000u) | (uint32_t)On);
-              ch[vi] = slotP ? ((chv & 0xFFFF0000u) | (uint32_t)Mn) : ((chv & 0xFFFFu) | ((uint32_t)Mn << 16));
-              cc.set(pi, newP, sx);
-              cc.set(vi, newV, sd);
-              if (On >= m) par[On - m] = (uint16_t)Pn;
-              if (Mn >= m) par[Mn - m] = (uint16_t)v;
-            }
-          }
+        if (tsa_team_has_rule(w.x, m)) {
+          const TsaTeamMove o = tsa_team_visit<W, MODE, SLICE>(P, lab, ch, cc, S, s_lse, s_ilse, T_, w, beta, t, [](int, int) {});
           if (t == 0) {
             np++;
-            na += acc;
+            na += o.acc;
+            if (o.acc && o.On >= m) par[o.On - m] = (uint16_t)o.Pn;
+            if (o.acc && o.Mn >= m) par[o.Mn - m] = (uint16_t)v;
           }
         }
         if (t == 0) {

@@ -23,6 +23,7 @@ hipError_t tsa_launch_team_full(const TsaLaunch& L, int mode, const TsaKParams& 
 // from five chains per unit on two waves keep all of them resident (sat70, 2048 chains: 6.9 ms against 10.2 with four).
 void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, TsaLaunch* L) {
   L->team = L->team_float = L->team_full = 0;
+  L->team_pre = want != 1 && tsa_team_pre_fits(P, lds_max);
   if (want == 1 || want > 8 || P.par_follow || P.par_band > 0) return;
   // the most LDS any launch of the context asks for: a float mode's cache, the level loop, slice moves
   const bool moves = P.slicing && P.slice_moves > 0;
