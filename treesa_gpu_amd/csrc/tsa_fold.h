@@ -42,11 +42,16 @@ __device__ __forceinline__ float tsa_node_eval(const TsaKParams& P, const uint64
 // set.  The lse chain of a lane is serial; its operands are read TSA_FOLD_BATCH at a time ahead of it, so that no
 // step waits on a load, and the size statistics run in a loop of their own.
 #define TSA_FOLD_BATCH 8
-// Rows [row0, row1) of the serial part: node 32 * row + l32 of each row folded into acc.
+// Rows [row0, row1) of the serial part: node 32 * row + l32 of each row folded into acc (from -inf, which row 0 starts
+// from, lse gives the cost itself).
 template <class FC>
 __device__ __forceinline__ float tsa_fold_rows(FC cost, int nint, const TsaMathTabs& T, int l32, float acc, int row0,
                                                int row1) {
   const int end = 32 * row1 < nint ? 32 * row1 : nint;
+  if (row0 == 0) {
+    if (l32 < end) acc = cost(l32) + 0.0f;
+    row0 = 1;
+  }
   for (int i0 = 32 * row0 + l32; i0 < end; i0 += 32 * TSA_FOLD_BATCH) {
     float cb[TSA_FOLD_BATCH];
 #pragma unroll
@@ -87,18 +92,15 @@ __device__ __forceinline__ TsaEvalOut tsa_fold_finish(const TsaKParams& P, FZ si
     }
   }
   int scmax = scl;
-  for (int o = 16; o > 0; o >>= 1) {
-    acc = tsa_lse_f(acc, __shfl_xor(acc, o, 32), T);
-    const int t = __shfl_xor(scmax, o, 32);
-    scmax = scmax > t ? scmax : t;
-  }
+  tsa_lane_butterfly<32>([&](auto o) {
+    acc = tsa_lse_f(acc, tsa_lane_xor<decltype(o)::value>(acc), T);
+  });
+  scmax = tsa_lane_max<32>(scmax);
   int cnt = (scl == scmax) ? cntl : 0, ns = 0;
   if (S)
     for (int w = l32; w < NW; w += 32) ns += __popcll(S[w]);
-  for (int o = 16; o > 0; o >>= 1) {
-    cnt += __shfl_xor(cnt, o, 32);
-    ns += __shfl_xor(ns, o, 32);
-  }
+  cnt = tsa_lane_sum<32>(cnt);
+  if (S) ns = tsa_lane_sum<32>(ns);
   int sc = scmax > P.leaf_sc ? scmax : P.leaf_sc;
   if (S && P.leaf_sc > scmax) {  // a leaf may be the largest tensor: masked leaf sizes
     int ll = 0;
@@ -107,10 +109,7 @@ __device__ __forceinline__ TsaEvalOut tsa_fold_finish(const TsaKParams& P, FZ si
       for (int w = 0; w < NW; w++) Z += __popcll(lf[(size_t)i * NW + w] & ~S[w]);
       ll = ll > Z ? ll : Z;
     }
-    for (int o = 16; o > 0; o >>= 1) {
-      const int t = __shfl_xor(ll, o, 32);
-      ll = ll > t ? ll : t;
-    }
+    ll = tsa_lane_max<32>(ll);
     sc = scmax > ll ? scmax : ll;
   }
   TsaEvalOut e;

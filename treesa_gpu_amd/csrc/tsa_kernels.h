@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 #include "tsa_arith.h"
+#include "tsa_lanes.h"
 #include "tsa_select.h"
 
 // Everything a kernel reads besides pointers, passed by value.

@@ -234,18 +234,15 @@ __device__ TsaEvalOut tsa_eval32(const TsaKParams& P, const uint64_t* lab, const
     }
   }
   int scmax = scl;
-  for (int o = 16; o > 0; o >>= 1) {
-    acc = tsa_lse_f(acc, __shfl_xor(acc, o, 32), T);
-    const int t = __shfl_xor(scmax, o, 32);
-    scmax = scmax > t ? scmax : t;
-  }
+  tsa_lane_butterfly<32>([&](auto o) {
+    acc = tsa_lse_f(acc, tsa_lane_xor<decltype(o)::value>(acc), T);
+  });
+  scmax = tsa_lane_max<32>(scmax);
   int cnt = (scl == scmax) ? cntl : 0, ns = 0;
   if (S)
     for (int w = l32; w < NW; w += 32) ns += __popcll(S[w]);
-  for (int o = 16; o > 0; o >>= 1) {
-    cnt += __shfl_xor(cnt, o, 32);
-    ns += __shfl_xor(ns, o, 32);
-  }
+  cnt = tsa_lane_sum<32>(cnt);
+  if (S) ns = tsa_lane_sum<32>(ns);
   int sc = scmax > P.leaf_sc ? scmax : P.leaf_sc;
   if (S && P.leaf_sc > scmax) {  // a leaf may be the largest tensor: masked leaf sizes
     int ll = 0;
@@ -254,10 +251,7 @@ __device__ TsaEvalOut tsa_eval32(const TsaKParams& P, const uint64_t* lab, const
       for (int w = 0; w < NW; w++) Z += __popcll(lf[(size_t)i * NW + w] & ~S[w]);
       ll = ll > Z ? ll : Z;
     }
-    for (int o = 16; o > 0; o >>= 1) {
-      const int t = __shfl_xor(ll, o, 32);
-      ll = ll > t ? ll : t;
-    }
+    ll = tsa_lane_max<32>(ll);
     sc = scmax > ll ? scmax : ll;
   }
   TsaEvalOut e;

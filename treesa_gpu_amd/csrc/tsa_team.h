@@ -74,18 +74,11 @@ struct TsaTeamShape {
   static constexpr int WL = W >= G ? W / G : 1;
 };
 
-// x of the lane's neighbour in its pair / across its quad's pairs.
-__device__ __forceinline__ uint32_t tsa_dpp_xor1(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xf, 0xf, true);  // quad_perm [1, 0, 3, 2]
-}
-__device__ __forceinline__ uint32_t tsa_dpp_xor2(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xf, 0xf, true);  // quad_perm [2, 3, 0, 1]
-}
 template <int G>
 __device__ __forceinline__ uint32_t tsa_group_sum(uint32_t x) {
   static_assert(G == 1 || G == 2 || G == 4, "groups inside a quad");
-  if (G >= 2) x += tsa_dpp_xor1(x);
-  if (G >= 4) x += tsa_dpp_xor2(x);
+  if constexpr (G >= 2) x += tsa_lane_xor<1>(x);
+  if constexpr (G >= 4) x += tsa_lane_xor<2>(x);
   return x;
 }
 
@@ -205,11 +198,11 @@ __device__ __forceinline__ TsaTeamMove tsa_team_visit(const TsaKParams& P, uint6
     const int q = t & 1;
     const float mine = tsa_node_cost_i<MODE>(q ? pk[6] : pk[2], q ? pk[7] : pk[3], q ? pk[8] : pk[4], q ? pk[9] : pk[5],
                                              P.model, T, s_ilse);
-    const float other = __uint_as_float(tsa_dpp_xor1(__float_as_uint(mine)));
+    const float other = tsa_lane_xor<1>(mine);
     newP = q ? other : mine;
     newV = q ? mine : other;
     const float h = tsa_lse_f(q ? costP : newP, q ? costV : newV, T);
-    const float ho = __uint_as_float(tsa_dpp_xor1(__float_as_uint(h)));
+    const float ho = tsa_lane_xor<1>(h);
     const float dtc = q ? ho - h : h - ho;
     const int sc0 = szP > sd ? szP : sd, sc1 = sx > sd ? sx : sd, scm = sc0 > sc1 ? sc0 : sc1;
     const float pw = ((float)scm > P.model.sc_target) ? P.model.sc_weight : 0.0f;
@@ -258,13 +251,8 @@ __device__ __forceinline__ bool tsa_team_slice_step(const TsaKParams& P, const u
       ncand = z > scm ? 1 : ncand + (z == scm);
       scm = z > scm ? z : scm;
     }
-    int top = scm;
-    for (int o = 32; o > 0; o >>= 1) {
-      const int x = __shfl_xor(top, o, 64);
-      top = top > x ? top : x;
-    }
-    ncand = scm == top ? ncand : 0;
-    for (int o = 32; o > 0; o >>= 1) ncand += __shfl_xor(ncand, o, 64);
+    const int top = tsa_lane_max<64>(scm);
+    ncand = tsa_lane_sum<64>(scm == top ? ncand : 0);
 #pragma unroll
     for (int w = 0; w < W; w++) ns += __popcll(S[w]);
     const TsaU4 r1 = tsa_philox(TsaU4{0x10000u + 2u * (uint32_t)j, sw, chain, 0u}, P.key0, P.key1);
@@ -310,11 +298,12 @@ __device__ __forceinline__ bool tsa_team_slice_step(const TsaKParams& P, const u
           tsa_fold_finish(P, [&](int i) { return f.size(i); }, hi ? S2 : S, lf, W, T, lane & 31,
                           tsa_fold_rows([&](int i) { return f.cost(i); }, nint, T, lane & 31, -INFINITY, 0, (nint + 31) / 32));
       const float E = tsa_slice_energy(x, P);
-      const bool acc = tsa_metropolis(r2.x, beta, __shfl(E, 32, 64) - __shfl(E, 0, 64), T.exp2);
-      const int from = acc ? 32 : 0;
-      e.lcost = __shfl(x.lcost, from, 64);
-      e.sc = __shfl(x.sc, from, 64);
-      e.ns = __shfl(x.ns, from, 64);
+      const auto from_lane = [](float y, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(y), k)); };
+      const bool acc = tsa_metropolis(r2.x, beta, from_lane(E, 32) - from_lane(E, 0), T.exp2);
+      const int from = __builtin_amdgcn_readfirstlane(acc ? 32 : 0);
+      e.lcost = from_lane(x.lcost, from);
+      e.sc = __builtin_amdgcn_readlane(x.sc, from);
+      e.ns = __builtin_amdgcn_readlane(x.ns, from);
       if (lane == 0) *s_acc = acc;
     }
     __syncthreads();

@@ -71,11 +71,10 @@ __device__ __forceinline__ void counts_unpack(const uint32_t (&a)[TsaFlat<MODE>:
 // stays below 2^16: a label set has at most 2 * TSA_WIDE_CPL * 64 * 64 = 16384 labels.
 template <int G, int N>
 __device__ __forceinline__ void group_sum(uint32_t (&a)[N]) {
+  tsa_lane_butterfly<G>([&](auto o) {
 #pragma unroll
-  for (int o = G / 2; o > 0; o >>= 1) {
-#pragma unroll
-    for (int i = 0; i < N; i++) a[i] += (uint32_t)__shfl_xor((int)a[i], o, G);
-  }
+    for (int i = 0; i < N; i++) a[i] += tsa_lane_xor<decltype(o)::value>(a[i]);
+  });
 }
 
 __device__ __forceinline__ long long wide_wave_sum(long long x) {
@@ -287,14 +286,9 @@ __device__ __forceinline__ bool wide_slice_step(const TsaKParams& P, const uint6
         scm = z > scm ? z : scm;
       }
       for (int w = lane; w < W; w += 64) ns += __popcll(sl.S[w]);
-      int top = scm;
-      for (int o = 32; o > 0; o >>= 1) {
-        const int x = __shfl_xor(top, o, 64);
-        top = top > x ? top : x;
-        ns += __shfl_xor(ns, o, 64);
-      }
-      ncand = scm == top ? ncand : 0;
-      for (int o = 32; o > 0; o >>= 1) ncand += __shfl_xor(ncand, o, 64);
+      const int top = tsa_lane_max<64>(scm);
+      ns = tsa_lane_sum<64>(ns);
+      ncand = tsa_lane_sum<64>(scm == top ? ncand : 0);
       const TsaU4 r1 = tsa_philox(TsaU4{0x10000u + 2u * (uint32_t)j, sw, chain, 0u}, P.key0, P.key1);
       int type;  // 0 add, 1 remove, 2 swap
       if (ns == 0) type = 0;
@@ -373,11 +367,12 @@ __device__ __forceinline__ bool wide_slice_step(const TsaKParams& P, const uint6
                           tsa_fold_rows([&](int i) { return fc[i]; }, nint, T, lane & 31, -INFINITY, 0, (nint + 31) / 32));
       const float pen = (float)x.sc > P.model.sc_target ? P.model.sc_weight * ((float)x.sc - P.model.sc_target) : 0.0f;
       const float E = (float)x.ns + x.lcost + pen;
-      const bool acc = tsa_metropolis(r2.x, beta, __shfl(E, 32, 64) - __shfl(E, 0, 64), T.exp2);
-      const int from = acc ? 32 : 0;
-      e.lcost = __shfl(x.lcost, from, 64);
-      e.sc = __shfl(x.sc, from, 64);
-      e.ns = __shfl(x.ns, from, 64);
+      const auto from_lane = [](float y, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(y), k)); };
+      const bool acc = tsa_metropolis(r2.x, beta, from_lane(E, 32) - from_lane(E, 0), T.exp2);
+      const int from = __builtin_amdgcn_readfirstlane(acc ? 32 : 0);
+      e.lcost = from_lane(x.lcost, from);
+      e.sc = __builtin_amdgcn_readlane(x.sc, from);
+      e.ns = __builtin_amdgcn_readlane(x.ns, from);
       if (lane == 0) *s_acc = acc;
     }
     __syncthreads();

@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(SUMS || SLICE ? 512 : 1024) k_wide(TsaKParams 
       for (;;) {
         int i0 = 0;
         if (lane == 0) i0 = atomicAdd(&s_next, gpw);
-        i0 = __shfl(i0, 0, 64);
+        i0 = __builtin_amdgcn_readfirstlane(i0);
         if (i0 >= nk) break;  // uniform within the wave
         const int j = ke + Ke * (i0 + gsub);
         if (i0 + gsub < nk) {  // uniform within a lane group
@@ -533,11 +533,10 @@ __global__ void __launch_bounds__(SUMS || SLICE ? 512 : 1024) k_wide(TsaKParams 
                     }
                   }
                 }
-#pragma unroll
-                for (int o2 = G / 2; o2 > 0; o2 >>= 1) {
-                  xs0 |= (uint64_t)__shfl_xor((unsigned long long)xs0, o2, G);
-                  xs1 |= (uint64_t)__shfl_xor((unsigned long long)xs1, o2, G);
-                }
+                tsa_lane_butterfly<G>([&](auto o2) {
+                  xs0 |= tsa_lane_xor<decltype(o2)::value>(xs0);
+                  xs1 |= tsa_lane_xor<decltype(o2)::value>(xs1);
+                });
                 if (t == 0) {
                   // this workgroup's copy now (no other visit of the phase reads P's summary), the other
                   // workgroups' copies from HBM in their replay
