@@ -599,7 +599,9 @@ __global__ void __launch_bounds__(256, (LVL && ORDER == 0 && MODE == 0) ? 3 : 1)
   __shared__ float s_lse[64];
   __shared__ uint64_t s_exp2[32];
   __shared__ uint64_t s_S[8];  // helper mode, level loop: the slice set at a level's end, for wave 1's fold
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, wpb = blockDim.x >> 6;
+  // (the wave's number by readfirstlane: what follows from the chain alone -- its hashes, addresses and first Philox
+  // products -- is scalar then; par, tc mode, W = 2: 115 -> 84 VGPRs, 8192 chains of sat100 9.44 -> 9.28 ms)
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), wpb = blockDim.x >> 6;
   const int NW = W > 0 ? W : P.W;
   const int m = P.m, nint = P.nint, nint4 = (nint + 3) & ~3;
   // the small tables every proposal indexes per lane live in LDS
