@@ -16,6 +16,7 @@
 
 #include "treesa_hip.h"
 #include "tsa_kernels.h"
+#include "tsa_valid.h"
 
 // Snapshot slots of the overlapped selection: an evaluated level's sweep takes the slot that the selection of
 // nslots - 1 levels back read, so the host may enqueue that many levels ahead of the device.  Three slots for
@@ -284,28 +285,6 @@ extern "C" int tsa_layout(int32_t m, int32_t nlab, int32_t wide, tsa_layout_t* o
   L.chain_words = (L.s_off + L.W + 1) & ~1;
   *out = L;
   return TSA_OK;
-}
-
-// Every chain must be a binary tree over all 2m-1 nodes rooted at 2m-2 (ids < 2m-1, each node reached
-// once); the kernels index label sets with these ids.  Reference check: csrc/treesa_gpu.cu:1127-1145.
-static bool valid_tree(const uint32_t* ch, int m, std::vector<char>& seen, std::vector<int>& st) {
-  const int n = 2 * m - 1;
-  seen.assign(n, 0);
-  st.clear();
-  st.push_back(n - 1);
-  int cnt = 0;
-  while (!st.empty()) {
-    const int v = st.back();
-    st.pop_back();
-    if (v < 0 || v >= n || seen[v]) return false;
-    seen[v] = 1;
-    cnt++;
-    if (v >= m) {
-      st.push_back((int)(ch[v - m] >> 16));
-      st.push_back((int)(ch[v - m] & 0xFFFFu));
-    }
-  }
-  return cnt == n;
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -821,11 +800,10 @@ extern "C" int tsa_upload(tsa_ctx* ctx, const uint64_t* population) {
   TSA_HIP(ctx, join_split(ctx));
   TSA_HIP(ctx, flush_track_init(ctx));
   const tsa_layout_t& L = ctx->lay;
-  std::vector<char> seen;
-  std::vector<int> st;
+  TsaTreeCheck valid;
   for (int c = 0; c < ctx->nchains; c++) {
     const uint64_t* rec = population + (size_t)c * L.chain_words;
-    if (!valid_tree(reinterpret_cast<const uint32_t*>(rec + L.ch_off), L.m, seen, st))
+    if (!valid(reinterpret_cast<const uint32_t*>(rec + L.ch_off), L.m))
       return fail(ctx, TSA_ERR_ARG, "tsa_upload: chain " + std::to_string(c) + " is not a valid tree");
   }
   TSA_HIP(ctx, quiesce_track(ctx));
