@@ -75,7 +75,8 @@ typedef struct tsa_config_t {
   /* measured H100 model, log2 of the constants (csrc/treesa_gpu.cu:1466-1474) */
   float v2_l3launch, v2_lperm2, v2_lcc_bit, v2_lcc_cell, v2_ltc_bit, v2_ltc_pad, v2_ltc_out, v2_lsmall_cell;
   int32_t v2_small_rank;
-  /* wide kernel plan (0 = automatic): waves per workgroup (1..16), workgroups per chain (1..16) */
+  /* wide kernel plan (0 = automatic): waves per workgroup (1..16), workgroups per chain (1..16).  On contexts whose
+   * chains sit in LDS, wide_waves is the waves per chain of par sweeps (1: one, 2..8; 0 automatic) */
   int32_t wide_waves, wide_wgs;
   /* 1: every tsa_sweeps on the register-width path also leaves the energies of the swept population ready,
    * so that tsa_energy / tsa_track launch no energy kernel; for callers that evaluate after every level.  The
