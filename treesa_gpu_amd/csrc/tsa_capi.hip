@@ -1398,19 +1398,11 @@ static int loop_fits(tsa_ctx* ctx, int32_t order, bool* fits) {
   return TSA_OK;
 }
 
-extern "C" int tsa_track(tsa_ctx* ctx, int32_t level) {
-  if (!ctx) return fail(ctx, TSA_ERR_ARG, "tsa_track: null context");
-  if (ctx->track_levels == 0) return fail(ctx, TSA_ERR_ARG, "tsa_track: no tsa_track_begin");
+// tsa_track without the check of the session's kind: the energies and the selection of one level.  tsa_anneal's
+// launches per level call it, whichever way the session's other tsa_anneal calls ran.
+static int track_level(tsa_ctx* ctx, int32_t level) {
   TSA_HIP(ctx, flush_track_init(ctx));
   TSA_HIP(ctx, flush_resample(ctx));
-  if (level < 0 || level >= ctx->track_levels) return fail(ctx, TSA_ERR_ARG, "tsa_track: level out of range");
-  bool loop_session = ctx->track_kind == TRACK_ANNEAL;
-  if (!loop_session && ctx->anneal_blocks) {  // (a session whose levels tsa_anneal runs, whichever way it does)
-    const int rc = loop_fits(ctx, TSA_ORDER_PAR, &loop_session);
-    if (rc != TSA_OK) return rc;
-  }
-  if (loop_session)
-    return fail(ctx, TSA_ERR_ARG, "tsa_track: this tracking session runs its levels with tsa_anneal");
   ctx->track_kind = TRACK_LEVELS;
   ctx->tend_staged = false;
   TsaSelect S = ctx->sel;
@@ -1449,6 +1441,22 @@ extern "C" int tsa_track(tsa_ctx* ctx, int32_t level) {
                                 L.ch_off, L.s_off, L.W, L.nint, nullptr, ctx->d_track, ctx->d_trace, ctx->d_best,
                                 ctx->d_tpart, ctx->d_tdone, ctx->st, true));
   return TSA_OK;
+}
+
+extern "C" int tsa_track(tsa_ctx* ctx, int32_t level) {
+  if (!ctx) return fail(ctx, TSA_ERR_ARG, "tsa_track: null context");
+  if (ctx->track_levels == 0) return fail(ctx, TSA_ERR_ARG, "tsa_track: no tsa_track_begin");
+  TSA_HIP(ctx, flush_track_init(ctx));
+  TSA_HIP(ctx, flush_resample(ctx));
+  if (level < 0 || level >= ctx->track_levels) return fail(ctx, TSA_ERR_ARG, "tsa_track: level out of range");
+  bool loop_session = ctx->track_kind == TRACK_ANNEAL;
+  if (!loop_session && ctx->anneal_blocks) {  // (a session whose levels tsa_anneal runs, whichever way it does)
+    const int rc = loop_fits(ctx, TSA_ORDER_PAR, &loop_session);
+    if (rc != TSA_OK) return rc;
+  }
+  if (loop_session)
+    return fail(ctx, TSA_ERR_ARG, "tsa_track: this tracking session runs its levels with tsa_anneal");
+  return track_level(ctx, level);
 }
 
 extern "C" int tsa_track_end(tsa_ctx* ctx, int32_t* best_chain, int32_t* best_level, double* best_score,
@@ -1668,7 +1676,7 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
     for (int l = 0; l < nlevels; l++) {
       int rc = tsa_sweeps(ctx, order, betas[l], sw, niters[l]);
       sw += (uint32_t)niters[l];
-      if (rc == TSA_OK && evaluated[l]) rc = tsa_track(ctx, level0 + l);
+      if (rc == TSA_OK && evaluated[l]) rc = track_level(ctx, level0 + l);
       if (rc != TSA_OK) return rc;
     }
     return TSA_OK;
