@@ -1,0 +1,73 @@
+"""The choice between one wave and a team of waves per chain (csrc/tsa_team_rule.h) where each was measured faster by
+more than the runs differ: MI355X, 256 compute units, 8 sweeps or fewer per launch and the energies after it."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SWEEPS, BLOCK, LOOP = range(3)
+# nodes, 64-bit words per label set
+TREES = {"sat4": (16, 1), "sat30": (127, 1), "sat60": (255, 1), "sat100": (425, 2), "reg60": (59, 2), "sq10": (99, 4),
+         "sq14": (195, 8), "reg250": (249, 8)}
+
+
+@pytest.fixture(scope="module")
+def waves(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rule") / "rule")
+    subprocess.run(["g++", "-O1", "-I", os.path.join(HERE, "..", "treesa_gpu_amd", "csrc"),
+                    os.path.join(HERE, "team_rule_check.cpp"), "-o", exe], check=True)
+
+    def run(tree, chains, nsweeps, kind=SWEEPS, mode=0, moves=False, asked=0):
+        nint, W = TREES[tree]
+        lanes = max(1, W // 2)
+        line = [asked, -(-chains // 256), nint * lanes // 64, nint * max(2, lanes) // 64, nint, int(moves), mode, kind, nsweeps]
+        return int(subprocess.run([exe], input=" ".join(map(str, line)), capture_output=True, text=True, check=True).stdout)
+
+    return run
+
+
+@pytest.mark.parametrize("tree,chains,nsweeps", [
+    ("sat4", 2048, 1), ("sat30", 3072, 1), ("sat60", 4096, 1), ("sat100", 2048, 1), ("reg60", 4096, 2), ("sq10", 4096, 1),
+    ("sat30", 4096, 4), ("sat100", 3072, 4)])
+def test_one_wave_for_few_sweeps_of_many_chains(waves, tree, chains, nsweeps):
+    assert waves(tree, chains, nsweeps) == 1
+
+
+@pytest.mark.parametrize("tree,chains,nsweeps", [
+    ("sat4", 64, 1), ("sat100", 1024, 1), ("sat30", 1536, 2), ("sat30", 2048, 4), ("sat60", 3072, 4), ("sat100", 4096, 8),
+    ("reg250", 4096, 1), ("sq14", 3072, 1), ("sq10", 3072, 8)])
+def test_team_where_its_start_pays(waves, tree, chains, nsweeps):
+    assert waves(tree, chains, nsweeps) > 1
+
+
+def test_two_waves_where_four_are_idle(waves):
+    assert waves("reg60", 1024, 1) == 2 and waves("sat100", 1024, 1) == 4
+
+
+def test_loop_keeps_every_chain_resident(waves):
+    for tree in ("sat4", "sat30", "sat60", "sat100"):
+        assert waves(tree, 3072, 10, LOOP) == 1
+        assert waves(tree, 3072, 10, LOOP, moves=True) > 1
+    assert waves("sat30", 2048, 10, LOOP) == 2 and waves("sq14", 3072, 10, LOOP) == 4
+
+
+@pytest.mark.parametrize("tree,chains", [("sat30", 2048), ("sat60", 8192), ("reg60", 4096), ("sq10", 4096)])
+def test_float_modes_two_waves_for_small_trees(waves, tree, chains):
+    for mode in (1, 2):
+        assert waves(tree, chains, 4, mode=mode) == 2
+    assert waves("sat100", chains, 4, mode=1) == 4
+
+
+def test_measured_time_model_of_tiny_trees(waves):
+    assert waves("sat4", 4096, 1, mode=2) == 1 and waves("sat4", 4096, 1, mode=1) == 2
+
+
+@pytest.mark.parametrize("chains,tree,want", [(72, "sat100", 8), (1024, "sat60", 4), (2048, "sat60", 2), (4096, "sat100", 4),
+                                              (6144, "sat100", 1)])
+def test_blocks_of_levels(waves, chains, tree, want):
+    assert waves(tree, chains, 8, BLOCK) == want
+
+
+def test_asked(waves):
+    assert [waves("sat30", 8192, 1, asked=a) for a in (2, 3, 8)] == [2, 3, 8]

@@ -118,6 +118,7 @@ struct tsa_ctx {
   // previous launch, so that the two halves of the population run their levels independently (the snapshot
   // slots keep them within a few levels of each other)
   bool fork_needed = true;
+  int par_waves = 0;           // waves per chain of the last par launch of the LDS kernels (0: none yet)
   long long split_levels = 0;  // sweep calls run as two launches (reported by tsa_describe)
   hipEvent_t ev_sweep[TSA_SNAP_MAX] = {};  // (the stop events of those sweeps' timing pairs)
   hipEvent_t ev_track[TSA_SNAP_MAX] = {};
@@ -541,9 +542,8 @@ extern "C" int tsa_create(const tsa_layout_t* lay, const uint64_t* leaf, int32_t
              lay->W, c->wide.G, c->wide.nsw, c->wide.nt / 64, c->wide.K, c->wide.smem, c->wide.eK, c->wide.fold_stage,
              c->wide.nxcd);
   else
-    snprintf(kb, sizeof kb, "%s W=%d waves/block=%d lds_bytes/wave=%d%s%s%s", use_lds ? "lds" : "global",
+    snprintf(kb, sizeof kb, "%s W=%d waves/block=%d lds_bytes/wave=%d%s%s", use_lds ? "lds" : "global",
              use_lds ? c->Wt : lay->W, c->L.wpb, c->L.lds_words * 8,
-             c->L.team > 0 ? (" par_team_waves=" + std::to_string(c->L.team)).c_str() : "",
              cfg->fused_energy && c->fold_apart ? " fold=apart" : "",
              c->L.draw_waves ? " preorder_draw_waves=3" : "");
   c->kname = kb;
@@ -1005,6 +1005,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
   } else {
     ctx->costs_valid = false;
     ctx->sums_valid = false;
+    if (!pre) ctx->par_waves = tsa_par_waves(ctx->L, ctx->mode, ctx->P, blk ? TSA_TEAM_BLOCK : TSA_TEAM_SWEEPS, nsweeps);
     const bool fuse = ctx->cfg.fused_energy != 0;
     const bool apart = fuse && (ctx->fold_apart || blk);  // (a block's costs are folded apart)
     // a split level: chains [0, h) on st, [h, nchains) on st3 (h in whole workgroups)
@@ -1389,7 +1390,7 @@ static int loop_fits(tsa_ctx* ctx, int32_t order, bool* fits) {
   if (r < 0) {
     TsaLevels q{};
     TsaLaunch one = ctx->L;
-    one.team = one.team_float = one.team_pre = 0;
+    one.team_fits = one.team_pre = 0;
     const TsaEnergyOut eo{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     TSA_HIP(ctx, tsa_launch_sweeps(one, ctx->mode, order, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix, ctx->nchains,
                                    0.0f, 0u, 0, ctx->d_stats, eo, ctx->st, nullptr, nullptr, &q, &r));
@@ -1766,6 +1767,8 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
     lv.best_words = ctx->lay.chain_words;
   }
   const TsaEnergyOut eo{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  if (order == TSA_ORDER_PAR)
+    ctx->par_waves = tsa_par_waves(ctx->L, ctx->mode, ctx->P, TSA_TEAM_LOOP, lv.total / lv.nlev);
   if (markers) TSA_HIP(ctx, hipEventRecord(e0, ctx->st));
   TSA_HIP(ctx, tsa_launch_sweeps(ctx->L, ctx->mode, order, ctx->P, ctx->d_rec, ctx->d_leaf, ctx->d_fix, n, 0.0f,
                                  sweep0, 0, ctx->d_stats, eo, ctx->st, markers ? nullptr : e0,
@@ -1890,7 +1893,12 @@ extern "C" int tsa_describe(tsa_ctx* ctx, char* buf, int32_t len) {
   char an[40] = "";
   if (ctx->lv_used == 2) snprintf(an, sizeof an, " anneal=level_blocks%d", ctx->blocks_k);
   else if (ctx->lv_used >= 0) snprintf(an, sizeof an, "%s", ctx->lv_used ? " anneal=level_loop" : " anneal=level_launches");
-  snprintf(buf, (size_t)len, "%s%s%s", ctx->kname.c_str(), sp, an);
+  char tm[32] = "";
+  if (ctx->L.lds && ctx->L.team_fits) {
+    const int w = ctx->par_waves > 0 ? ctx->par_waves : tsa_team_waves(ctx->L.team_rule, ctx->mode, TSA_TEAM_BLOCK, 1);
+    if (w > 1) snprintf(tm, sizeof tm, " par_team_waves=%d", w);
+  }
+  snprintf(buf, (size_t)len, "%s%s%s%s", ctx->kname.c_str(), tm, sp, an);
   return TSA_OK;
 }
 

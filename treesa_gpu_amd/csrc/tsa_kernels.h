@@ -7,6 +7,7 @@
 #include "tsa_arith.h"
 #include "tsa_lanes.h"
 #include "tsa_select.h"
+#include "tsa_team_rule.h"
 
 // Everything a kernel reads besides pointers, passed by value.
 struct TsaKParams {
@@ -71,9 +72,11 @@ struct TsaLaunch {
   int lds_words;     // LDS words per wave
   int draw_waves;    // 1: pre-order sweeps run one chain per workgroup with helper waves that draw ahead
   int lds_max;       // dynamic LDS bytes a workgroup may have, less the kernel's static LDS
-  // par sweeps of a chain in LDS: waves per chain of k_team in tc mode and in the float modes (0: k_sweep, one wave
-  // per chain), and whether its work-list entries are the long ones
-  int team, team_float, team_full;
+  // par sweeps of a chain in LDS: whether k_team can run them, how its waves are chosen, whether its work-list entries
+  // are the long ones, and (set by tsa_launch_sweeps) the waves of this launch
+  int team_fits;
+  TsaTeamRule team_rule;
+  int team_full, team;
   int team_pre;      // pre-order sweeps with helper waves (draw_waves) run k_team_pre
 };
 
@@ -186,6 +189,8 @@ hipError_t tsa_launch_sweeps_sliced(const TsaLaunch& L, int mode, int order, con
                                     const uint64_t* leaf, const uint32_t* fix, int nchains, float beta, uint32_t sweep0,
                                     int nsweeps, unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st,
                                     hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res);
+// Waves per chain of a par launch of the LDS kernels (1: k_sweep); nsweeps as tsa_team_waves takes it.
+int tsa_par_waves(const TsaLaunch& L, int mode, const TsaKParams& P, TsaTeamKind kind, int nsweeps);
 // Par sweeps with L.team waves per chain (tsa_team.h): work-list entries long (L.team_full) or short, without and with
 // slicing; res as above.
 hipError_t tsa_launch_team_full(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,

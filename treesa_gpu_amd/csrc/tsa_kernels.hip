@@ -259,16 +259,25 @@ __global__ void __launch_bounds__(256) k_track_init(TsaTrackState* st, unsigned 
 // ---------------------------------------------------------------------------------------------------
 // The kernels without slice code (sets never masked) are instantiated here, the slicing ones in
 // tsa_sweep_sliced.hip.
+int tsa_par_waves(const TsaLaunch& L, int mode, const TsaKParams& P, TsaTeamKind kind, int nsweeps) {
+  // (the team's visits take the costs before a move from a cache whose operands are in slot order, so its model may
+  // not tell left from right: the gpu model does when m0 and n0 differ)
+  if (!L.lds || !L.team_fits || (mode == 1 && P.model.m0 != P.model.n0)) return 1;
+  return tsa_team_waves(L.team_rule, mode, kind, nsweeps);
+}
 hipError_t tsa_launch_sweeps(const TsaLaunch& L, int mode, int order, const TsaKParams& P, uint64_t* rec,
                              const uint64_t* leaf, const uint32_t* fix, int nchains, float beta, uint32_t sweep0,
                              int nsweeps, unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st,
                              hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res) {
-  // (the team's visits take the costs before a move from a cache whose operands are in slot order, so its model may
-  // not tell left from right: the gpu model does when m0 and n0 differ)
-  if ((mode == 0 ? L.team : L.team_float) > 0 && L.lds && order == 0 && (mode != 1 || P.model.m0 == P.model.n0)) {
+  const int waves = order != 0 ? 1
+                    : lv       ? tsa_par_waves(L, mode, P, TSA_TEAM_LOOP, lv->nlev > 0 ? lv->total / lv->nlev : 0)
+                               : tsa_par_waves(L, mode, P, eo.blk.n > 0 ? TSA_TEAM_BLOCK : TSA_TEAM_SWEEPS, nsweeps);
+  if (waves > 1) {
+    TsaLaunch T = L;
+    T.team = waves;
     const auto go = P.slicing ? (L.team_full ? tsa_launch_team_sliced_full : tsa_launch_team_sliced_compact)
                               : (L.team_full ? tsa_launch_team_full : tsa_launch_team_compact);
-    return go(L, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
+    return go(T, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
   }
   if (L.team_pre && L.lds && L.draw_waves && order == 1 && !P.slicing && (mode != 1 || P.model.m0 == P.model.n0))
     return tsa_launch_team_pre(L.W, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);

@@ -702,7 +702,7 @@ static hipError_t launch_team_t(const TsaLaunch& L, const TsaKParams& P, uint64_
                                 hipEvent_t e1, const TsaLevels* lv, int* res) {
   const int caches = tsa_team_caches(SLICE && P.slice_moves > 0, LVL);
   const size_t smem = (size_t)tsa_team_lds(P.m, P.nint, W, P.chain_words, MODE, caches, FULL).bytes;
-  const int threads = 64 * (MODE == 0 ? L.team : L.team_float);
+  const int threads = 64 * L.team;
   const void* const fn = reinterpret_cast<const void*>(&k_team<W, MODE, SLICE, LVL, FULL>);
   if (smem > 65536) {
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
