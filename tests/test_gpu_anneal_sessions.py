@@ -1,5 +1,7 @@
 """One tracking session whose tsa_anneal calls run in different ways (blocks of levels in par order, launches per level
-in pre-order) against tsa_sweeps + tsa_track per level, bit for bit."""
+in pre-order) against tsa_sweeps + tsa_track per level, bit for bit; and that the call only enqueues."""
+import time
+
 import numpy as np
 import pytest
 
@@ -52,3 +54,25 @@ def test_orders_in_one_session(orders, mode):
         want = finish(ctx)
     for k, (a, b) in enumerate(zip(got, want)):
         np.testing.assert_array_equal(a, b, err_msg=f"output {k}")
+
+
+def test_anneal_is_enqueued():
+    """With every chain resident tsa_anneal returns while the device still has most of the schedule before it: no level
+    waits for the host, however many blocks of levels the schedule has."""
+    levels, niters = 400, 60
+    inst = network("sat", 30)
+    betas = np.linspace(0.1, 9.0, levels).astype(np.float32)
+    with start(inst, 48) as ctx:
+        for warm in (True, False):
+            ctx.track_begin("tc", sc_target=8.0, max_levels=levels)
+            ctx.wait()
+            t0 = time.perf_counter()
+            ctx.anneal(capi.ORDER_PAR, betas, [niters] * levels, [1] * levels)
+            t1 = time.perf_counter()
+            ctx.wait()
+            t2 = time.perf_counter()
+            ctx.track_end()
+        assert "anneal=level_blocks" in ctx.describe()
+    print(f"[gpu] enqueued in {1e3 * (t1 - t0):.1f} of {1e3 * (t2 - t0):.1f} ms", flush=True)
+    assert t1 - t0 < 0.5 * (t2 - t0)
+

@@ -147,6 +147,7 @@ struct tsa_ctx {
   // dispatch (about 6 us of host time) rather than in the dispatch itself (about 20 us).
   bool host_waited = false;
   int track_kind = 0;
+  bool anneal_async = false;   // this session's sweeps wait for their snapshot slots on the device, not on the host
   bool anneal_blocks = false;  // tsa_anneal ran this session's levels in blocks where it would have run the loop
   bool lv_reset = false;
   int lv_resident[6] = {-1, -1, -1, -1, -1, -1};  // level-loop chains resident per compute unit, per mode and order
@@ -753,10 +754,22 @@ static int ensure_slots(tsa_ctx* ctx, int n) {
 // for it (it ran beside the previous sweep, which is still queued or running, so the device does not idle)
 // rather than putting a wait on the stream: a cross-stream wait in the queue costs about 10 us per level
 // even when it is already satisfied, and the host is normally many levels ahead of the device.
-static hipError_t claim_slot(tsa_ctx* c, int s) {
-  hipError_t e = hipSuccess;
-  if (c->track_pending[s]) e = hipEventSynchronize(c->ev_track[c->track_ev[s]]);
+// In a session whose levels the level loop could have run (anneal_async) the wait goes on the streams that sweep, so
+// that tsa_anneal enqueues its whole schedule as the loop does, unless it is satisfied already; waited: the event that
+// the streams were made to wait for last (a block's slots share one).
+static hipError_t claim_slot(tsa_ctx* c, int s, hipEvent_t* waited) {
+  if (!c->track_pending[s]) return hipSuccess;
   c->track_pending[s] = false;
+  const hipEvent_t ev = c->ev_track[c->track_ev[s]];
+  if (!c->anneal_async) return hipEventSynchronize(ev);
+  if (ev == *waited) return hipSuccess;
+  hipError_t e = hipEventQuery(ev);
+  if (e == hipErrorNotReady) {
+    (void)hipGetLastError();
+    e = hipStreamWaitEvent(c->st, ev, 0);
+    if (e == hipSuccess && c->st3) e = hipStreamWaitEvent(c->st3, ev, 0);
+  }
+  *waited = ev;
   return e;
 }
 
@@ -912,6 +925,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
     return fail(ctx, TSA_ERR_ARG, "block of levels on the wide path: one workgroup per chain, the overlapped "
                                   "selection with the fold apart, tc mode, par order");
   const bool pre = order == TSA_ORDER_PREORDER;
+  hipEvent_t waited = nullptr;  // (claim_slot)
   if (ctx->wide.on && (!pre || ctx->wide_pre)) {
     TSA_HIP(ctx, join_split(ctx));
     TSA_HIP(ctx, flush_resample(ctx));
@@ -957,7 +971,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
         blk_slots[i] = -1;
         if (!blk_ev[i]) continue;
         const int t = ctx->slot;
-        TSA_HIP(ctx, claim_slot(ctx, t));
+        TSA_HIP(ctx, claim_slot(ctx, t, &waited));
         ctx->snap_kind[t] = SNAP_WIDE;
         sy.blk_ch[i] = ctx->d_snap_ch[t];
         sy.blk_cost[i] = ctx->d_snap_cost[t];
@@ -967,7 +981,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
       }
     } else if (ctx->overlap) {
       s = ctx->slot;
-      TSA_HIP(ctx, claim_slot(ctx, s));
+      TSA_HIP(ctx, claim_slot(ctx, s, &waited));
       sy.snap_ch = ctx->d_snap_ch[s];
       if (snap_fold) {
         sy.flc = reinterpret_cast<float*>(ctx->d_snap_en[s]);
@@ -1034,7 +1048,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
         eo.blk.ch[i] = nullptr;
         if (!blk_ev[i]) continue;
         const int t = ctx->slot;
-        TSA_HIP(ctx, claim_slot(ctx, t));
+        TSA_HIP(ctx, claim_slot(ctx, t, &waited));
         ctx->snap_kind[t] = SNAP_COSTS;
         eo.blk.cost[i] = ctx->d_snap_cost[t];
         eo.blk.z[i] = ctx->d_snap_nz[t];
@@ -1046,7 +1060,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
       // node costs (or, folded in the kernel, energies) and children words go to snapshot slot s, folded and
       // selected on st2 by tsa_track
       s = ctx->slot;
-      TSA_HIP(ctx, claim_slot(ctx, s));
+      TSA_HIP(ctx, claim_slot(ctx, s, &waited));
       ctx->snap_kind[s] = apart ? SNAP_COSTS : SNAP_ENERGIES;
       if (apart) {
         eo.cost = ctx->d_snap_cost[s];
@@ -1272,7 +1286,7 @@ extern "C" int tsa_track_begin(tsa_ctx* ctx, const tsa_select_t* sel, int32_t ma
   ctx->overlap = want_overlap;
   ctx->slot = 0;
   ctx->track_kind = 0;
-  ctx->anneal_blocks = false;
+  ctx->anneal_blocks = ctx->anneal_async = false;
   ctx->lv_reset = true;
   ctx->lv_evaluated.assign((size_t)max_levels, 0);
   static_assert(sizeof(TsaTraceRowD) % 8 == 0, "trace rows are whole words");
@@ -1615,37 +1629,36 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
   if (ctx->cfg.level_blocks < 0 || ctx->cfg.level_blocks > TSA_BLOCK_MAX)
     return fail(ctx, TSA_ERR_ARG, "tsa_config_t.level_blocks: 0 (automatic) or 1..8");
   const int K = ctx->cfg.level_blocks > 0 ? ctx->cfg.level_blocks : TSA_BLOCK_MAX;
-  // One launch for the whole call when the context's kernels run the level loop (the LDS kernels), it is not
-  // turned off, and either it is asked for or every chain of it is resident at once: with more chains than
-  // that, a chain resident only after others have run all their levels would leave the per-level launches'
-  // fold of every chain in one round and their occupancy for nothing.  A session that began with one kind
-  // stays with it (the best is tracked per chain by the level loop, per level by tsa_track).
+  // Blocks of levels (par order, the overlapped selection): several levels per sweep launch, each evaluated level
+  // leaving its snapshot in a slot of its own, whose fold and selection tsa_track runs as for one level.  The folds of a
+  // block run beside the next block's sweeps on lanes of their own, where the level loop's chains fold serially
+  // between their levels (40 levels of one sweep: 72 chains of sat100 1.03 -> 0.55 ms, 768 1.41 -> 0.80, 3072 4.17 ->
+  // 1.88); and with more chains than the device holds at once a block of levels has one tail, in which fewer and fewer
+  // chains are left to run, for all of them.
+  // Else one launch for the whole call, the level loop, when the context's kernels run it (the LDS kernels), it is not
+  // turned off, and either it is asked for or every chain of it is resident at once: with more chains than that, a
+  // chain resident only after others have run all their levels would leave the per-level launches' fold of every chain
+  // in one round and their occupancy for nothing.  A session that began with the loop stays with it (it tracks the best
+  // per chain, the others per level).
   bool loop = ctx->track_kind == TRACK_ANNEAL;
-  if (ctx->track_kind == 0 && !ctx->wide.on && ctx->L.lds && ctx->cfg.level_loop >= 0) {
-    // ... or blocks of levels run instead: their folds of a level's energies run beside the next block's sweeps on
-    // lanes of their own, where the loop's chains fold serially between their levels (par order, 40 levels of one
-    // sweep: 72 chains of sat100 1.03 -> 0.55 ms, 768 1.41 -> 0.80, 3072 4.17 -> 1.88)
-    loop = ctx->cfg.level_loop > 0;
-    if (!loop) {
-      ctx->anneal_blocks = lds_blocks_ok(ctx, order, K);
-      if (!ctx->anneal_blocks) {
-        const int rc = loop_fits(ctx, order, &loop);
-        if (rc != TSA_OK) return rc;
-      }
-    }
+  const bool choose = ctx->track_kind == 0 && !ctx->wide.on && ctx->L.lds && ctx->cfg.level_loop >= 0;
+  if (choose) loop = ctx->cfg.level_loop > 0;
+  const bool wide_blocks = !loop && K > 1 && wide_blocks_ok(ctx, order);
+  const bool blocks = wide_blocks || (!loop && lds_blocks_ok(ctx, order, K));
+  if (choose && !loop) ctx->anneal_blocks = blocks;
+  if (blocks && ensure_slots(ctx, 3 * K) != TSA_OK) return TSA_ERR_HIP;
+  if (choose && !loop) {
+    bool fits = false;
+    const int rc = loop_fits(ctx, order, &fits);
+    if (rc != TSA_OK) return rc;
+    if (blocks) ctx->anneal_async = fits;
+    else loop = fits;
   }
   ctx->lv_used = loop ? 1 : 0;
   // (a pending session start: the first sweeps enqueue it, or the level loop's set-up launch does it)
-  // Several levels per sweep launch (the one-wave LDS kernels with the overlapped selection and the fold apart,
-  // where the population is more than twice what the device holds at once): a launch ends with a tail in which
-  // fewer and fewer chains are left to run, and a level of one sweep per chain is short next to it; a block of
-  // levels has one tail for all of them.  Each evaluated level of a block leaves its snapshot in a slot of its
-  // own, whose fold and selection tsa_track runs as for one level.
-  const bool wide_blocks = !loop && K > 1 && wide_blocks_ok(ctx, order);
-  if (wide_blocks || (!loop && lds_blocks_ok(ctx, order, K))) {
+  if (blocks) {
     ctx->lv_used = 2;
     ctx->blocks_k = K;
-    if (ensure_slots(ctx, 3 * K) != TSA_OK) return TSA_ERR_HIP;
     uint32_t sw = sweep0;
     for (int l = 0; l < nlevels; l += K) {
       TsaBlock blk{};
