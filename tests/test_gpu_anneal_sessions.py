@@ -1,5 +1,9 @@
 """One tracking session whose tsa_anneal calls run in different ways (blocks of levels in par order, launches per level
-in pre-order) against tsa_sweeps + tsa_track per level, bit for bit; and that the call only enqueues."""
+in pre-order) against tsa_sweeps + tsa_track per level, bit for bit; that the call only enqueues; and that it runs
+without memory for the blocks' snapshots."""
+import os
+import subprocess
+import sys
 import time
 
 import numpy as np
@@ -76,3 +80,50 @@ def test_anneal_is_enqueued():
     print(f"[gpu] enqueued in {1e3 * (t1 - t0):.1f} of {1e3 * (t2 - t0):.1f} ms", flush=True)
     assert t1 - t0 < 0.5 * (t2 - t0)
 
+
+SHIM = """
+#include <dlfcn.h>
+#include <stddef.h>
+static size_t limit = 0;
+extern "C" void shim_limit(size_t n) { limit = n; }
+extern "C" int hipMalloc(void** p, size_t n) {
+  static int (*real)(void**, size_t) = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
+  if (limit && n >= limit) {
+    *p = nullptr;
+    return 2;  // hipErrorOutOfMemory
+  }
+  return real(p, n);
+}
+"""
+NO_ROOM = """
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # found before the runtime's own by the library's calls
+import numpy as np
+from test_gpu_anneal_sessions import LEVELS, NITERS, finish, start
+from test_gpu_team import network
+from treesa_gpu_amd import capi
+out = []
+for limit in (1 << 18, 0):
+    with start(network("sat", 30), 48) as ctx:
+        ctx.track_begin("tc", sc_target=8.0, max_levels=LEVELS)
+        shim.shim_limit(ctypes.c_size_t(limit))
+        ctx.anneal(capi.ORDER_PAR, np.linspace(0.1, 9.0, LEVELS).astype(np.float32), [NITERS] * LEVELS, [1] * LEVELS)
+        shim.shim_limit(ctypes.c_size_t(0))
+        out.append(finish(ctx))
+        print(ctx.describe(), flush=True)
+for a, b in zip(*out):
+    np.testing.assert_array_equal(a, b)
+"""
+
+
+def test_anneal_without_room_for_the_blocks_snapshots(tmp_path):
+    """Where the blocks' snapshots cannot be allocated the call runs the level loop, which needs none."""
+    (tmp_path / "shim.cpp").write_text(SHIM)
+    lib = str(tmp_path / "libshim.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", str(tmp_path / "shim.cpp"), "-o", lib, "-ldl"], check=True)
+    here = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([here, os.path.dirname(here), os.environ.get("PYTHONPATH", "")]))
+    p = subprocess.run([sys.executable, "-c", NO_ROOM, lib], capture_output=True, text=True, timeout=100, env=env)
+    print(p.stdout, p.stderr[-2000:], flush=True)
+    assert p.returncode == 0
+    assert [w.split("anneal=")[1] for w in p.stdout.strip().splitlines()] == ["level_loop", "level_blocks8"]

@@ -1644,9 +1644,13 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
   const bool choose = ctx->track_kind == 0 && !ctx->wide.on && ctx->L.lds && ctx->cfg.level_loop >= 0;
   if (choose) loop = ctx->cfg.level_loop > 0;
   const bool wide_blocks = !loop && K > 1 && wide_blocks_ok(ctx, order);
-  const bool blocks = wide_blocks || (!loop && lds_blocks_ok(ctx, order, K));
+  bool blocks = wide_blocks || (!loop && lds_blocks_ok(ctx, order, K));
   if (choose && !loop) ctx->anneal_blocks = blocks;
-  if (blocks && ensure_slots(ctx, 3 * K) != TSA_OK) return TSA_ERR_HIP;
+  if (blocks && ensure_slots(ctx, 3 * K) != TSA_OK) {
+    if (wide_blocks || ctx->fold_apart) return TSA_ERR_HIP;
+    (void)hipGetLastError();  // no room for the blocks' snapshots: the ways that do without
+    blocks = ctx->anneal_blocks = false;
+  }
   if (choose && !loop) {
     bool fits = false;
     const int rc = loop_fits(ctx, order, &fits);
