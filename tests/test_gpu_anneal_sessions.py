@@ -60,6 +60,23 @@ def test_orders_in_one_session(orders, mode):
         np.testing.assert_array_equal(a, b, err_msg=f"output {k}")
 
 
+@pytest.mark.parametrize("chains", [48, 1100])
+def test_levels_one_by_one(chains):
+    """A call of one level is a launch of its own, in a session with blocks of levels before and after it."""
+    inst = network("sat", 30)
+    betas = np.linspace(0.1, 9.0, LEVELS).astype(np.float32)
+    out = []
+    for cut in ((0, 1, 6, 7, 8, LEVELS), (0, LEVELS)):
+        with start(inst, chains) as ctx:
+            ctx.track_begin("tc", sc_target=8.0, max_levels=LEVELS)
+            for l0, l1 in zip(cut, cut[1:]):
+                ctx.anneal(capi.ORDER_PAR, betas[l0:l1], [NITERS] * (l1 - l0), [1] * (l1 - l0), level0=l0, sweep0=l0 * NITERS)
+                assert ("anneal=level_launches" if l1 - l0 == 1 else "anneal=level_blocks") in ctx.describe()
+            out.append(finish(ctx))
+    for k, (a, b) in enumerate(zip(*out)):
+        np.testing.assert_array_equal(a, b, err_msg=f"output {k}")
+
+
 def test_anneal_is_enqueued():
     """With every chain resident tsa_anneal returns while the device still has most of the schedule before it: no level
     waits for the host, however many blocks of levels the schedule has."""

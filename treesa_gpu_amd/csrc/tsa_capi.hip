@@ -1646,6 +1646,10 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
   const bool wide_blocks = !loop && K > 1 && wide_blocks_ok(ctx, order);
   bool blocks = wide_blocks || (!loop && lds_blocks_ok(ctx, order, K));
   if (choose && !loop) ctx->anneal_blocks = blocks;
+  // One level has no next block beside which its fold could run: a launch that folds in the sweep kernel (sat30, 16
+  // chains, one sweep: 55 us against 59 .. 66 as a block; 1024 chains 62 against 93).
+  const bool single = blocks && !wide_blocks && !ctx->fold_apart && nlevels == 1;
+  if (single) blocks = false;
   if (blocks && ensure_slots(ctx, 3 * K) != TSA_OK) {
     if (wide_blocks || ctx->fold_apart) return TSA_ERR_HIP;
     (void)hipGetLastError();  // no room for the blocks' snapshots: the ways that do without
@@ -1655,7 +1659,7 @@ extern "C" int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t n
     bool fits = false;
     const int rc = loop_fits(ctx, order, &fits);
     if (rc != TSA_OK) return rc;
-    if (blocks) ctx->anneal_async = fits;
+    if (blocks || single) ctx->anneal_async = fits;
     else loop = fits;
   }
   ctx->lv_used = loop ? 1 : 0;
