@@ -17,6 +17,7 @@
 #include "treesa_hip.h"
 #include "tsa_kernels.h"
 #include "tsa_valid.h"
+#include "tsa_wide_rule.h"
 
 // Snapshot slots of the overlapped selection: an evaluated level's sweep takes the slot that the selection of
 // nslots - 1 levels back read, so the host may enqueue that many levels ahead of the device.  Three slots for
@@ -697,6 +698,13 @@ static TendLayout tend_layout(const tsa_ctx* c) {
   return o;
 }
 
+// Whether a context's sweeps in this order run on the lane groups of the wide path (else k_sweep on sets in HBM).
+static bool wide_runs(const tsa_ctx* c, bool pre) {
+  if (!c->wide.on) return false;
+  if (pre) return c->wide_pre && tsa_wide_pre_pays(c->mode, c->lay.W, c->nchains, c->ncu);
+  return !c->cfg.slicing || tsa_wide_slice_pays(c->mode, c->lay.W, c->nchains, c->ncu);
+}
+
 // The wide path's overlapped selection with the fold in the sweep launch: dense plans of one workgroup per chain
 // with more chains than compute units (with fewer, the fold of the node-cost snapshot runs beside the next
 // sweep as well).
@@ -926,7 +934,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
                                   "selection with the fold apart, tc mode, par order");
   const bool pre = order == TSA_ORDER_PREORDER;
   hipEvent_t waited = nullptr;  // (claim_slot)
-  if (ctx->wide.on && (!pre || ctx->wide_pre)) {
+  if (wide_runs(ctx, pre)) {
     TSA_HIP(ctx, join_split(ctx));
     TSA_HIP(ctx, flush_resample(ctx));
     // energies stay a separate fold of the node-cost cache: every chain ends its sweep at about the same
