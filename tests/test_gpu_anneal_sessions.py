@@ -77,6 +77,27 @@ def test_levels_one_by_one(chains):
         np.testing.assert_array_equal(a, b, err_msg=f"output {k}")
 
 
+def test_levels_run_again():
+    """A session's levels run three times over: every block claims the slots of the same levels' earlier selections."""
+    inst, levels = network("sat", 30), 5
+    betas = np.linspace(0.1, 9.0, levels).astype(np.float32)
+    out = []
+    for blocks in (True, False):
+        with start(inst, 48) as ctx:
+            ctx.track_begin("tc", sc_target=8.0, max_levels=levels)
+            for again in range(3):
+                sweep = again * levels * NITERS
+                if blocks:
+                    ctx.anneal(capi.ORDER_PAR, betas, [NITERS] * levels, [1] * levels, sweep0=sweep)
+                    continue
+                for lev in range(levels):
+                    ctx.sweeps(capi.ORDER_PAR, betas[lev], sweep + lev * NITERS, NITERS)
+                    ctx.track(lev)
+            out.append(finish(ctx))
+    for k, (a, b) in enumerate(zip(*out)):
+        np.testing.assert_array_equal(a, b, err_msg=f"output {k}")
+
+
 def test_anneal_is_enqueued():
     """With every chain resident tsa_anneal returns while the device still has most of the schedule before it: no level
     waits for the host, however many blocks of levels the schedule has."""
