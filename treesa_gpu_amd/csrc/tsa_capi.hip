@@ -119,6 +119,7 @@ struct tsa_ctx {
   // previous launch, so that the two halves of the population run their levels independently (the snapshot
   // slots keep them within a few levels of each other)
   bool fork_needed = true;
+  bool one_lane = false;       // the last sweeps of a wide context ran one lane per proposal (tsa_wide_rule.h, or slicing)
   int par_waves = 0;           // waves per chain of the last par launch of the LDS kernels (0: none yet)
   long long split_levels = 0;  // sweep calls run as two launches (reported by tsa_describe)
   hipEvent_t ev_sweep[TSA_SNAP_MAX] = {};  // (the stop events of those sweeps' timing pairs)
@@ -935,6 +936,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
   const bool pre = order == TSA_ORDER_PREORDER;
   hipEvent_t waited = nullptr;  // (claim_slot)
   if (wide_runs(ctx, pre)) {
+    ctx->one_lane = false;
     TSA_HIP(ctx, join_split(ctx));
     TSA_HIP(ctx, flush_resample(ctx));
     // energies stay a separate fold of the node-cost cache: every chain ends its sweep at about the same
@@ -1027,6 +1029,7 @@ static int sweeps_impl(tsa_ctx* ctx, int32_t order, float beta, uint32_t sweep0,
   } else {
     ctx->costs_valid = false;
     ctx->sums_valid = false;
+    ctx->one_lane = ctx->wide.on;
     if (!pre) ctx->par_waves = tsa_par_waves(ctx->L, ctx->mode, ctx->P, blk ? TSA_TEAM_BLOCK : TSA_TEAM_SWEEPS, nsweeps);
     const bool fuse = ctx->cfg.fused_energy != 0;
     const bool apart = fuse && (ctx->fold_apart || blk);  // (a block's costs are folded apart)
@@ -1924,10 +1927,20 @@ extern "C" int tsa_describe(tsa_ctx* ctx, char* buf, int32_t len) {
   char an[40] = "";
   if (ctx->lv_used == 2) snprintf(an, sizeof an, " anneal=level_blocks%d", ctx->blocks_k);
   else if (ctx->lv_used >= 0) snprintf(an, sizeof an, "%s", ctx->lv_used ? " anneal=level_loop" : " anneal=level_launches");
-  char tm[32] = "";
-  if (ctx->L.lds && ctx->L.team_fits) {
-    const int w = ctx->par_waves > 0 ? ctx->par_waves : tsa_team_waves(ctx->L.team_rule, ctx->mode, TSA_TEAM_BLOCK, 1);
-    if (w > 1) snprintf(tm, sizeof tm, " par_team_waves=%d", w);
+  char tm[96] = "";
+  if (ctx->wide.on) {
+    if (ctx->one_lane) snprintf(tm, sizeof tm, " sweeps=one_lane");
+    else if (wide_runs(ctx, true))
+      snprintf(tm, sizeof tm, " preorder_lanes=%d preorder_waves=%d", tsa_wide_pre_lanes(ctx->lay.W),
+               tsa_wide_pre_waves(ctx->nchains, ctx->ncu));
+  } else if (ctx->L.lds) {
+    const int lanes = tsa_team_lanes(ctx->L.W, ctx->mode);
+    const int w = !ctx->L.team_fits ? 1 : ctx->par_waves > 0 ? ctx->par_waves
+                  : tsa_team_waves(ctx->L.team_rule, ctx->mode, TSA_TEAM_BLOCK, 1);
+    int at = 0;
+    if (w > 1) at = snprintf(tm, sizeof tm, " par_team_waves=%d team_lanes=%d team_entries=%s", w, lanes,
+                             ctx->L.team_full ? "long" : "short");
+    if (tsa_pre_team(ctx->L, ctx->mode, ctx->P)) snprintf(tm + at, sizeof tm - at, " preorder_lanes=%d", lanes);
   }
   snprintf(buf, (size_t)len, "%s%s%s%s", ctx->kname.c_str(), tm, sp, an);
   return TSA_OK;

@@ -191,6 +191,8 @@ hipError_t tsa_launch_sweeps_sliced(const TsaLaunch& L, int mode, int order, con
                                     hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res);
 // Waves per chain of a par launch of the LDS kernels (1: k_sweep); nsweeps as tsa_team_waves takes it.
 int tsa_par_waves(const TsaLaunch& L, int mode, const TsaKParams& P, TsaTeamKind kind, int nsweeps);
+// Whether pre-order sweeps run k_team_pre.
+bool tsa_pre_team(const TsaLaunch& L, int mode, const TsaKParams& P);
 // Par sweeps with L.team waves per chain (tsa_team.h): work-list entries long (L.team_full) or short, without and with
 // slicing; res as above.
 hipError_t tsa_launch_team_full(const TsaLaunch& L, int mode, const TsaKParams& P, uint64_t* rec, const uint64_t* leaf,
@@ -217,7 +219,7 @@ hipError_t tsa_launch_team_pre(int W, int mode, const TsaKParams& P, uint64_t* r
                                unsigned long long* stats, const TsaEnergyOut& eo, hipStream_t st, hipEvent_t e0,
                                hipEvent_t e1, const TsaLevels* lv, int* res);
 // L's team fields for par sweeps of nchains chains with lds_max bytes of LDS per workgroup.  want: 0 automatic, 1 one
-// wave, 2..8 that many.
+// wave, 2..8 that many (more: automatic).
 void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, TsaLaunch* L);
 hipError_t tsa_launch_energy(int Wt, int mode, const TsaKParams& P, const uint64_t* rec, const uint64_t* leaf,
                              const uint32_t* fix, int nchains, float* lc, int* sc, int* ns, hipStream_t st);
@@ -436,6 +438,10 @@ hipError_t tsa_launch_wide(const TsaWide& X, int mode, const TsaKParams& P, uint
                            const uint32_t* fix, int nchains, float beta, uint32_t sweep0, int nsweeps,
                            unsigned long long* stats, const TsaWideSync& sy, hipStream_t st,
                            hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+// k_wide_pre's lanes per proposal: as many as a set has chunks, up to two chunks a lane (fewer, fuller lanes only lengthen
+// the step); its waves per chain: a full frontier of 64 nodes in one round where a compute unit has one chain.
+static inline int tsa_wide_pre_lanes(int W) { return W / 2 <= 32 ? 16 : W / 2 <= 64 ? 32 : 64; }
+static inline int tsa_wide_pre_waves(int nchains, int ncu) { return nchains <= ncu ? 16 : 8; }
 // Pre-order sweeps of wide chains without slicing (tsa_wide_pre.hip), the node-cost cache of X exact before (tc mode) and
 // kept; whether the context's chains fit it (lds_max: LDS bytes per workgroup).
 bool tsa_wide_pre_fits(const TsaKParams& P, int lds_max);

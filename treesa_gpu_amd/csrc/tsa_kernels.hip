@@ -259,10 +259,14 @@ __global__ void __launch_bounds__(256) k_track_init(TsaTrackState* st, unsigned 
 // ---------------------------------------------------------------------------------------------------
 // The kernels without slice code (sets never masked) are instantiated here, the slicing ones in
 // tsa_sweep_sliced.hip.
+// (the team's visits take the costs before a move from a cache whose operands are in slot order, so its model may
+// not tell left from right: the gpu model does when m0 and n0 differ)
+static bool team_model(int mode, const TsaKParams& P) { return mode != 1 || P.model.m0 == P.model.n0; }
+bool tsa_pre_team(const TsaLaunch& L, int mode, const TsaKParams& P) {
+  return L.team_pre && L.lds && L.draw_waves && !P.slicing && team_model(mode, P);
+}
 int tsa_par_waves(const TsaLaunch& L, int mode, const TsaKParams& P, TsaTeamKind kind, int nsweeps) {
-  // (the team's visits take the costs before a move from a cache whose operands are in slot order, so its model may
-  // not tell left from right: the gpu model does when m0 and n0 differ)
-  if (!L.lds || !L.team_fits || (mode == 1 && P.model.m0 != P.model.n0)) return 1;
+  if (!L.lds || !L.team_fits || !team_model(mode, P)) return 1;
   return tsa_team_waves(L.team_rule, mode, kind, nsweeps);
 }
 hipError_t tsa_launch_sweeps(const TsaLaunch& L, int mode, int order, const TsaKParams& P, uint64_t* rec,
@@ -279,7 +283,7 @@ hipError_t tsa_launch_sweeps(const TsaLaunch& L, int mode, int order, const TsaK
                               : (L.team_full ? tsa_launch_team_full : tsa_launch_team_compact);
     return go(T, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
   }
-  if (L.team_pre && L.lds && L.draw_waves && order == 1 && !P.slicing && (mode != 1 || P.model.m0 == P.model.n0))
+  if (order == 1 && tsa_pre_team(L, mode, P))
     return tsa_launch_team_pre(L.W, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
   if (P.slicing)
     return tsa_launch_sweeps_sliced(L, mode, order, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st,

@@ -45,7 +45,7 @@ __host__ __device__ static inline TsaTeamLds tsa_team_lds(int m, int nint, int W
   L.bytes = (b + 15) & ~15;
   return L;
 }
-#define TSA_TEAM_STATIC_LDS 4096  // room for k_team's static LDS (under 3.5 KB)
+#define TSA_TEAM_STATIC_LDS 4096  // room for the static LDS of k_team and k_team_pre
 // Copies of the cache a launch needs: the chain's, the proposed slice set's, and the level being folded.
 static inline int tsa_team_caches(bool slice_moves, bool levels) { return 1 + (slice_moves ? 1 : 0) + (levels ? 1 : 0); }
 
@@ -70,7 +70,7 @@ struct TsaTeamCache {
 // Lanes per proposal and label words per lane: two words a lane; the float modes always two lanes or more.
 template <int W, int MODE>
 struct TsaTeamShape {
-  static constexpr int G = W <= 2 ? (MODE == 0 ? 1 : 2) : W / 2;
+  static constexpr int G = tsa_team_lanes(W, MODE);
   static constexpr int WL = W >= G ? W / G : 1;
 };
 
@@ -357,6 +357,8 @@ __global__ void __launch_bounds__(512, MODE == 0 ? 4 : 2)
   __shared__ uint64_t s_S[8], s_S2[8];  // the slice set being folded; the proposed one
   __shared__ int s_cnt[2], s_draw, s_acc;
   __shared__ __align__(16) unsigned char s_fold[LVL ? sizeof(TsaTeamFold) : 16];
+  static_assert(sizeof s_lse + sizeof s_ilse + sizeof s_mt + sizeof s_S + sizeof s_S2 + 16 + sizeof(TsaTeamFold) + 64 <=
+                    TSA_TEAM_STATIC_LDS, "the plan leaves TSA_TEAM_STATIC_LDS bytes to the static arrays");
   constexpr int G = TsaTeamShape<W, MODE>::G, WL = TsaTeamShape<W, MODE>::WL;
   const int tid = threadIdx.x, NT = blockDim.x, T = NT >> 6, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -11,8 +11,9 @@ hipError_t tsa_launch_team_full(const TsaLaunch& L, int mode, const TsaKParams& 
 
 void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int want, TsaLaunch* L) {
   L->team_fits = L->team_full = 0;
+  if (want > 8) want = 0;  // (a plan for the wide kernel: it says nothing here)
   L->team_pre = want != 1 && tsa_team_pre_fits(P, lds_max);
-  if (want == 1 || want > 8 || P.par_follow || P.par_band > 0) return;
+  if (want == 1 || P.par_follow || P.par_band > 0) return;
   // the most LDS any launch of the context asks for: a float mode's cache, the level loop, slice moves
   const bool moves = P.slicing && P.slice_moves > 0;
   const int caches = tsa_team_caches(moves, true);
@@ -21,8 +22,7 @@ void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int w
   // long entries save a visit two dependent LDS round trips; they may not cost a compute unit a chain
   const int most = tsa_team_lds(P.m, P.nint, P.W, P.chain_words, 1, caches, 1).bytes + TSA_TEAM_STATIC_LDS;
   L->team_full = most <= lds_max && (long long)most * per_cu <= lds_max;
-  const int lanes = P.W <= 2 ? 1 : P.W / 2;  // of a proposal (the float modes: two or more)
   L->team_fits = 1;
-  L->team_rule = TsaTeamRule{want > 0 ? want : 0, per_cu, P.nint * lanes / 64, P.nint * (lanes < 2 ? 2 : lanes) / 64, P.nint,
-                             moves};
+  L->team_rule = TsaTeamRule{want > 0 ? want : 0, per_cu, P.nint * tsa_team_lanes(P.W, 0) / 64,
+                             P.nint * tsa_team_lanes(P.W, 1) / 64, P.nint, moves};
 }

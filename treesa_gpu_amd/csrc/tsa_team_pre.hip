@@ -42,6 +42,8 @@ __global__ void __launch_bounds__(64 * (1 + TSA_DRAW_HELPERS))
   __shared__ float s_lse[64], s_ilse[TSA_ILSE];
   __shared__ uint64_t s_mt[TSA_MT_WORDS];
   __shared__ __align__(16) unsigned char s_fold[LVL ? sizeof(TsaTeamFold) : 16];
+  static_assert(sizeof s_lse + sizeof s_ilse + sizeof s_mt + sizeof(TsaTeamFold) + 64 <= TSA_TEAM_STATIC_LDS,
+                "the plan leaves TSA_TEAM_STATIC_LDS bytes to the static arrays");
   constexpr int G = TsaTeamShape<W, MODE>::G, GPW = 64 / G, R = G;  // R rounds of GPW proposals hold a step's 64
   const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -10,6 +10,8 @@ struct TsaTeamRule {
   int nint;
   bool moves;               // slice moves
 };
+// Lanes of a proposal: two 64-bit words of its label sets a lane; the float modes always two lanes or more.
+static constexpr int tsa_team_lanes(int W, int mode) { return W <= 2 ? (mode == 0 ? 1 : 2) : W / 2; }
 // A launch of sweeps at one beta, a block of levels, the level loop.
 enum TsaTeamKind { TSA_TEAM_SWEEPS, TSA_TEAM_BLOCK, TSA_TEAM_LOOP };
 

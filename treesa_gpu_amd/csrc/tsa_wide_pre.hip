@@ -188,11 +188,7 @@ hipError_t tsa_launch_wide_pre(int mode, const TsaKParams& P, uint64_t* rec, con
                                int nchains, int ncu, float beta, uint32_t sweep0, int nsweeps,
                                unsigned long long* stats, const TsaWideSync& sy, hipStream_t st, hipEvent_t e0,
                                hipEvent_t e1) {
-  const int nch = P.W / 2;
-  // as many lanes as a set has chunks, up to two chunks a lane: fewer, fuller lanes only lengthen the step
-  const int G = nch <= 32 ? 16 : nch <= 64 ? 32 : 64;
-  // a full frontier of 64 nodes in one round where a compute unit has one chain
-  const int threads = nchains <= ncu ? 1024 : 512;
+  const int G = tsa_wide_pre_lanes(P.W), threads = 64 * tsa_wide_pre_waves(nchains, ncu);
 #define TSA_PRE_GO(G)                                                                                                    \
   return mode == 0   ? launch_pre<G, 0>(threads, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, sy, st, e0, e1) \
          : mode == 1 ? launch_pre<G, 1>(threads, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, sy, st, e0, e1) \

@@ -58,11 +58,14 @@ class Device {
  public:
   Device(const tsa_layout_t& lay, const std::vector<uint64_t>& leaf, int leaf_sc, const tsa_config_t& cfg,
          int nchains) {
-    if (tsa_create(&lay, leaf.data(), leaf_sc, &cfg, nchains, &ctx_) != TSA_OK) {
-      const std::string msg = tsa_last_error(nullptr);
-      if (msg.find("fit") != std::string::npos)
-        throw DeviceError("chains do not fit in shared memory (try --kernel warp / --lpc 32)");
-      throw DeviceError("treesa_hip: " + msg);
+    create(lay, leaf, leaf_sc, cfg, nchains);
+    if (cfg.wide_waves > 0 && describe().compare(0, 3, "lds") == 0) {
+      // --wpc plans the wide kernel; where chains sit in LDS it has no effect
+      tsa_destroy(ctx_);
+      ctx_ = nullptr;
+      tsa_config_t automatic = cfg;
+      automatic.wide_waves = 0;
+      create(lay, leaf, leaf_sc, automatic, nchains);
     }
   }
   ~Device() { tsa_destroy(ctx_); }
@@ -88,6 +91,14 @@ class Device {
   }
 
  private:
+  void create(const tsa_layout_t& lay, const std::vector<uint64_t>& leaf, int leaf_sc, const tsa_config_t& cfg,
+              int nchains) {
+    if (tsa_create(&lay, leaf.data(), leaf_sc, &cfg, nchains, &ctx_) == TSA_OK) return;
+    const std::string msg = tsa_last_error(nullptr);
+    if (msg.find("fit") != std::string::npos)
+      throw DeviceError("chains do not fit in shared memory (try --kernel warp / --lpc 32)");
+    throw DeviceError("treesa_hip: " + msg);
+  }
   tsa_ctx* ctx_ = nullptr;
 };
 
@@ -718,14 +729,18 @@ int Run::anneal() {
   static const char* counter_keys[7] = {"proposals",       "accepts",       "warp_steps", "node_visits",
                                         "slice_proposals", "slice_accepts", "busy_lanes"};
   for (int k = 0; k < 7; k++) j.integer(counter_keys[k], (long long)st[k]);
-  // the visit mapping in the reference's terms: lanes per proposal (coop_*), waves per chain (wpc) and the
-  // proposals one round of a chain's waves holds (lpc: 64 on the one-wave kernels, waves x 64 / G on the wide
-  // kernel).  warp_steps counts what the reference's kernels count (csrc/treesa_gpu.cu:716, 990): rounds of
+  // the visit mapping of the last sweeps in the reference's terms: lanes per proposal (coop_*), waves that visit for a
+  // chain (wpc) and the proposals one of their rounds holds (lpc: waves x 64 / lanes in par order, a step's 64 nodes in
+  // pre-order).  warp_steps counts what the reference's kernels count (csrc/treesa_gpu.cu:716, 990): rounds of
   // up to lpc visits in pre-order, phases in par order; so node_visits / (lpc * warp_steps) is the lane
   // occupancy of a pre-order sweep and the visits per phase and visit slot of a par sweep, as there
   // (bench/throughput.py:68).
-  const int G = desc_int(desc, " G=", 1);
-  const int wpc = desc.compare(0, 5, "wide ") == 0 ? desc_int(desc, " waves/block=", 1) * desc_int(desc, " blocks/chain=", 1) : 1;
+  const bool wide = desc.compare(0, 5, "wide ") == 0 && desc.find(" sweeps=one_lane") == std::string::npos;
+  const bool par = order_ == TSA_ORDER_PAR;
+  const int G = !par ? desc_int(desc, " preorder_lanes=", 1) : desc_int(desc, wide ? " G=" : " team_lanes=", 1);
+  const int wpc = !par   ? desc_int(desc, " preorder_waves=", 1)
+                  : wide ? desc_int(desc, " waves/block=", 1) * desc_int(desc, " blocks/chain=", 1)
+                         : desc_int(desc, " par_team_waves=", 1);
   j.integer("coop_max", G);
   j.integer("coop_min", G);
   j.integer("coop_full", G);
@@ -742,7 +757,7 @@ int Run::anneal() {
   j.integer("nw", nw32);
   j.integer("W64", lay_.W);
   j.integer("word_bits", 64);
-  j.integer("lpc", wpc * 64 / G);
+  j.integer("lpc", par ? wpc * 64 / G : 64);
   j.text("kernel", kernel_label());
   j.text("hip_kernel", desc);
   j.text("scheme", O_.scheme);
