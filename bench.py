@@ -262,9 +262,6 @@ def cpu_port_worker(cfgname, nsample, level_loop_out=None):
     O = orc.Oracle(m, nlab, ixs, iy)
     ocfg = capi.make_config(mode="tc", sc_target=C["sc_target"], seed=1, slicing=C["slicing"], slice_moves=1)
     P = orc.params_from_config(ocfg, inst.leaf_sc, nlab)
-    sample_out = None
-    if level_loop_out and not C["slicing"]:
-        level_loop_out, sample_out = None, level_loop_out  # independent chains: the first nsample ones stand alone
     if level_loop_out:
         p0 = oracle_population(O, lay, m, C["nchains"], 1, trees)
         nlev = len(betas)
@@ -279,10 +276,7 @@ def cpu_port_worker(cfgname, nsample, level_loop_out=None):
     t0 = time.perf_counter()
     for lev, b in enumerate(betas):
         O.sweeps(P, lay, p0, order, b, lev * C["niters"], C["niters"])
-    secs = time.perf_counter() - t0
-    if sample_out:
-        np.save(sample_out, p0)
-    print(secs)
+    print(time.perf_counter() - t0)
 
 
 def sample_slots(nchains, n):
@@ -382,20 +376,6 @@ def cpu_baseline(cfgname, C, inst, lay, trees, betas, nsample, dump=None, gpu=No
                     (parity["accepts"][0] != parity["accepts"][1])
         where = " and ".join(f"{c0}..{c0 + k - 1}" for c0, k in ranges)
         sample = (f"{n_all} chains (chain slots {where} of this workload's start) x {len(betas) * C['niters']} "
-                  f"sweeps on {threads} threads: {n_all * per_level:.3e} visits in {secs:.1f} s")
-    elif not C["slicing"]:
-        # no harness: the oracle port on the first chains of the workload.  An eighth
-        # of the harness's sample: c2's whole population takes 49 s at the port's 1.4e7 visits/s on 16 cores, this 3 s
-        kind = "port"
-        nsample = max(1, nsample // 8)
-        n_all = min(C["nchains"], nsample * threads)
-        with tempfile.TemporaryDirectory() as td:
-            out = os.path.join(td, "port_pop.npy")
-            secs = port_run(cfgname, n_all, threads, out if dump else None)
-            if dump:
-                parity = parity_of(lay, inst.nlab, load_population(dump, C["nchains"], lay)[:n_all], port_pop=np.load(out))
-        secs1 = port_run(cfgname, nsample, 1)
-        sample = (f"{n_all} chains (chain slots 0..{n_all - 1} of this workload's start) x {len(betas) * C['niters']} "
                   f"sweeps on {threads} threads: {n_all * per_level:.3e} visits in {secs:.1f} s")
     else:
         kind = "port"
