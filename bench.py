@@ -20,8 +20,8 @@ event-timed sweep kernels only.
 
 roofline: of the sweep kernel, per launch, with the resource that bounds it.  Where the binary runs the level
 loop in one launch (scheme indep with every chain resident at once: c1) a launch is the whole schedule
-(levels_per_launch); where it sweeps blocks of K levels per launch (scheme indep with more than twice the chains
-the device holds at once: c2, "anneal=level_blocksK") a launch is K levels (the schedule's last block may be
+(levels_per_launch); where it sweeps blocks of K levels per launch (scheme indep in par order: c2,
+"anneal=level_blocksK") a launch is K levels (the schedule's last block may be
 shorter: the figures are averages over the run's launches, and the HBM traffic is the committed summary's per
 level times the levels per launch); else one level.  Chains staged in LDS (c1-c3):
 bound "lds", achieved = the algorithmic bytes of the proposals (5 label sets of W words + 8 B of children per
@@ -387,8 +387,8 @@ def cpu_baseline(cfgname, C, inst, lay, trees, betas, nsample, dump=None, gpu=No
             if dump:
                 parity = parity_of(lay, inst.nlab, load_population(dump, C["nchains"], lay), port_pop=np.load(out))
         secs1 = port_run(cfgname, nsample, 1)
-        sample = (f"{'the whole level loop (every chain, population annealing after every level)' if dump else ''}"
-                  f" {n_all} chains x {len(betas) * C['niters']} sweeps with slice moves on {threads} threads: "
+        sample = (f"{'the whole level loop (every chain' + (', population annealing after every level' if C['scheme'] == 'pa' else '') + ')' if dump else ''}"
+                  f" {n_all} chains x {len(betas) * C['niters']} sweeps{' with slice moves' if C['slicing'] else ''} on {threads} threads: "
                   f"{n_all * per_level:.3e} visits in {secs:.1f} s").strip()
     res = dict(value=n_all * per_level / secs, unit="node visits/s", cores=threads, kind=kind, sample=sample,
                one_core={"value": nsample * per_level / secs1, "sample": f"{nsample} chains, {secs1:.1f} s"},
