@@ -1042,8 +1042,8 @@ hipError_t tsa_wide_plan(const TsaKParams& P, int nchains, int want_waves, int w
   waves = waves < 1 ? 1 : (waves > max_waves ? max_waves : waves);
   X.nt = 64 * waves;
   const int band = P.par_band > 0 ? 1 : 0;
-  // dynamic LDS cap: the device maximum less room for the kernels' static LDS (under 1 KB today)
-  const int nint4 = (P.nint + 3) & ~3, lds_cap = lds_max - 4096;
+  // dynamic LDS cap: the device maximum less room for the kernels' static LDS (under 3 KB)
+  const int nint4 = (P.nint + 3) & ~3, lds_cap = lds_max - 4080;
   if (X.nsw) {  // the input tensors' summaries go to LDS too when they fit
     X.lsum_lds = tsa_wide_lds(P.nint, band, 0, X.nsw, P.m).bytes <= lds_cap ? 1 : 0;
     if (!X.lsum_lds && tsa_wide_lds(P.nint, band, 0, X.nsw, 0).bytes > lds_cap) {
