@@ -329,12 +329,15 @@ __global__ void __launch_bounds__(SUMS || SLICE ? 512 : 1024) k_wide(TsaKParams 
           }
         }
       };
-      const int wvs = __builtin_amdgcn_readfirstlane(wv);
-      for (int g0 = wvs; g0 < ngrp; g0 += 8 * nwv) {
-        if (g0 + 4 * nwv < ngrp) scan(TsaLaneStep<8>{}, g0);
-        else if (g0 + 2 * nwv < ngrp) scan(TsaLaneStep<4>{}, g0);
-        else if (g0 + nwv < ngrp) scan(TsaLaneStep<2>{}, g0);
-        else scan(TsaLaneStep<1>{}, g0);
+      if constexpr (SUMS) {  // (trees with sets this wide have groups for a full batch)
+        for (int g0 = wv; g0 < ngrp; g0 += 8 * nwv) scan(TsaLaneStep<8>{}, g0);
+      } else {
+        for (int g0 = __builtin_amdgcn_readfirstlane(wv); g0 < ngrp; g0 += 8 * nwv) {
+          if (g0 + 4 * nwv < ngrp) scan(TsaLaneStep<8>{}, g0);
+          else if (g0 + 2 * nwv < ngrp) scan(TsaLaneStep<4>{}, g0);
+          else if (g0 + nwv < ngrp) scan(TsaLaneStep<2>{}, g0);
+          else scan(TsaLaneStep<1>{}, g0);
+        }
       }
       __syncthreads();
       if constexpr (COOP) {
