@@ -8,8 +8,18 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 SWEEPS, BLOCK, LOOP = range(3)
 # nodes, 64-bit words per label set
-TREES = {"sat4": (16, 1), "sat30": (127, 1), "sat60": (255, 1), "sat100": (425, 2), "reg60": (59, 2), "sq10": (99, 4),
-         "sq14": (195, 8), "reg250": (249, 8)}
+TREES = {"sat4": (16, 1), "sat30": (127, 1), "sat60": (255, 1), "sat70": (297, 2), "sat100": (425, 2), "reg60": (59, 2),
+         "sq10": (99, 4), "sq12": (143, 8), "sq14": (195, 8), "reg250": (249, 8)}
+
+
+def resident(nint, W, per_cu):
+    """Chains that 160 KB of LDS hold: teams sweeping, teams in the loop, single waves (four to a workgroup)."""
+    n4, leaf, rec = (nint + 3) // 4 * 4, (nint + 1) * W * 8, nint * (W * 8 + 4) + W * 8
+    team = lambda entry, caches: leaf + rec + n4 * entry + 8 * n4 + 4 * n4 * caches + 4 * n4 + 32  # noqa: E731
+    long_entries = (team(16, 2) + n4 * 4 + 4096) * per_cu <= 163840  # (with a float mode's caches of 6 bytes)
+    entry = 16 if long_entries else 2
+    return (163840 // (team(entry, 1) + 2640), 163840 // (team(entry, 2) + 3392),
+            163840 // (leaf + 4 * (rec + 6 * n4 + 16) + 512) * 4)
 
 
 @pytest.fixture(scope="module")
@@ -21,7 +31,9 @@ def waves(tmp_path_factory):
     def run(tree, chains, nsweeps, kind=SWEEPS, mode=0, moves=False, asked=0):
         nint, W = TREES[tree]
         lanes = max(1, W // 2)
-        line = [asked, -(-chains // 256), nint * lanes // 64, nint * max(2, lanes) // 64, nint, int(moves), mode, kind, nsweeps]
+        per_cu = -(-chains // 256)
+        line = [asked, per_cu, nint * lanes // 64, nint * max(2, lanes) // 64, nint, int(moves), *resident(nint, W, per_cu), W,
+                mode, kind, nsweeps]
         return int(subprocess.run([exe], input=" ".join(map(str, line)), capture_output=True, text=True, check=True).stdout)
 
     return run
@@ -29,14 +41,14 @@ def waves(tmp_path_factory):
 
 @pytest.mark.parametrize("tree,chains,nsweeps", [
     ("sat4", 2048, 1), ("sat30", 3072, 1), ("sat60", 4096, 1), ("sat100", 2048, 1), ("reg60", 4096, 2), ("sq10", 4096, 1),
-    ("sat30", 4096, 4), ("sat100", 3072, 4)])
+    ("sat30", 4096, 4), ("sat100", 3072, 4), ("sq14", 2048, 1), ("sat70", 3072, 8), ("sat30", 4096, 8)])
 def test_one_wave_for_few_sweeps_of_many_chains(waves, tree, chains, nsweeps):
     assert waves(tree, chains, nsweeps) == 1
 
 
 @pytest.mark.parametrize("tree,chains,nsweeps", [
     ("sat4", 64, 1), ("sat100", 1024, 1), ("sat30", 1536, 2), ("sat30", 2048, 4), ("sat60", 3072, 4), ("sat100", 4096, 8),
-    ("reg250", 4096, 1), ("sq14", 3072, 1), ("sq10", 3072, 8)])
+    ("reg250", 4096, 1), ("sq14", 3072, 1), ("sq14", 2048, 2), ("sq10", 3072, 8)])
 def test_team_where_its_start_pays(waves, tree, chains, nsweeps):
     assert waves(tree, chains, nsweeps) > 1
 
@@ -46,10 +58,12 @@ def test_two_waves_where_four_are_idle(waves):
 
 
 def test_loop_keeps_every_chain_resident(waves):
-    for tree in ("sat4", "sat30", "sat60", "sat100"):
+    for tree in ("sat4", "sat30", "sat60", "sat100", "sq12"):
         assert waves(tree, 3072, 10, LOOP) == 1
         assert waves(tree, 3072, 10, LOOP, moves=True) > 1
+    assert waves("sat70", 2048, 5, LOOP) == 1 and waves("sat70", 1792, 5, LOOP) == 2
     assert waves("sat30", 2048, 10, LOOP) == 2 and waves("sq14", 3072, 10, LOOP) == 4
+    assert waves("sq12", 2048, 5, LOOP) == 1 and waves("sq12", 2048, 1, LOOP) == 4
 
 
 @pytest.mark.parametrize("tree,chains", [("sat30", 2048), ("sat60", 8192), ("reg60", 4096), ("sq10", 4096)])

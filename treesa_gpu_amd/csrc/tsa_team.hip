@@ -23,6 +23,11 @@ void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int w
   const int most = tsa_team_lds(P.m, P.nint, P.W, P.chain_words, 1, caches, 1).bytes + TSA_TEAM_STATIC_LDS;
   L->team_full = most <= lds_max && (long long)most * per_cu <= lds_max;
   L->team_fits = 1;
+  const auto chains = [&](bool loop, int fixed) {  // that LDS holds; fixed: the launch's static LDS
+    return lds_max / (tsa_team_lds(P.m, P.nint, P.W, P.chain_words, 0, tsa_team_caches(moves, loop), L->team_full).bytes + fixed);
+  };
+  const int one = (((P.m * P.W + 1) & ~1) + L->wpb * L->lds_words) * 8 + 512;  // a workgroup of k_sweep
   L->team_rule = TsaTeamRule{want > 0 ? want : 0, per_cu, P.nint * tsa_team_lanes(P.W, 0) / 64,
-                             P.nint * tsa_team_lanes(P.W, 1) / 64, P.nint, moves};
+                             P.nint * tsa_team_lanes(P.W, 1) / 64, P.nint, moves, chains(false, 2640), chains(true, 3392),
+                             lds_max / one * L->wpb, P.W};
 }

@@ -9,11 +9,20 @@ struct TsaTeamRule {
   int units, units_float;   // wavefuls of lanes that one proposal per node takes, in tc mode and in the float modes
   int nint;
   bool moves;               // slice moves
+  // chains that a compute unit's LDS holds: of a team's launch of sweeps and of its level loop, and of one wave each
+  int lds, lds_loop, lds_one;
+  int words;                // 64-bit words per label set
 };
 // Lanes of a proposal: two 64-bit words of its label sets a lane; the float modes always two lanes or more.
 static constexpr int tsa_team_lanes(int W, int mode) { return W <= 2 ? (mode == 0 ? 1 : 2) : W / 2; }
 // A launch of sweeps at one beta, a block of levels, the level loop.
 enum TsaTeamKind { TSA_TEAM_SWEEPS, TSA_TEAM_BLOCK, TSA_TEAM_LOOP };
+
+// Rounds of resident chains that per_cu chains take, at most `waves` and `lds` of them at once.
+static inline int tsa_rounds(int per_cu, int waves, int lds) {
+  const int most = waves < lds ? waves : lds;
+  return (per_cu + most - 1) / (most > 0 ? most : 1);
+}
 
 // The lines lie where the measured times cross (par order, blocks of levels, 40 levels of one sweep, us):
 //   chains  sat100: one wave / team of 2 / 4 / 8    sat60                     sq14 (8 words)
@@ -32,7 +41,7 @@ static inline int tsa_team_waves_tc(const TsaTeamRule& r, TsaTeamKind kind, int 
   if (r.per_cu <= 1) return 8;
   if (r.per_cu <= 4) {
     // (a launch whose trees do not fill four waves: 1024 chains of reg60, one sweep: 36.9 us, two waves 31.4)
-    if (kind == TSA_TEAM_SWEEPS && r.per_cu > 2 && r.units < 5) return 2;
+    if (kind == TSA_TEAM_SWEEPS && r.per_cu > 2 && r.units < 4) return 2;
     return 4;
   }
   // More chains than that per unit share it either way, and a team's launch starts with a pass over every chain for its
@@ -41,19 +50,32 @@ static inline int tsa_team_waves_tc(const TsaTeamRule& r, TsaTeamKind kind, int 
   //   one sweep     sat30   36.9 / 40.3   41.8 / 48.2   45.8 / 62.0     sat100  56.0 / 66.7   64.3 / 80.0   87.5 / 98.4
   //   two           sat30   47.2 / 47.7   54.2 / 56.8   60.1 / 73.1     sat100  76.3 / 82.4   89.3 / 103.7  121.6 / 128.7
   //   four          sat30   67.1 / 62.5   78.1 / 75.4   87.6 / 102.8    sat100  115.5 / 119.9 135.6 / 152.4 190.5 / 192.3
-  // Wide proposals (units >= 8) are ahead from the first (reg250: 92 / 70, 137 / 105, 170 / 123).
+  // And it takes more rounds where fewer teams than single waves are resident at once (28 waves of k_team a unit, 24 to 16
+  // of k_sweep, and the LDS): then two waves per chain are never ahead (sat70, 12 per unit, eight sweeps 206 / 248), four
+  // from eight sweeps on, and wide proposals (units >= 8) from two (sq14, 8 per unit, one sweep 87 / 97, two 110 / 111).
+  const int waves_one = r.words <= 2 ? 24 : r.words <= 4 ? 20 : 16;
+  const int rounds_one = tsa_rounds(r.per_cu, waves_one, r.lds_one);
   if (kind == TSA_TEAM_SWEEPS) {
     if (r.moves) return r.nint < 64 && nsweeps < 2 ? 1 : big;
-    if (r.units >= 8 || r.per_cu <= 6) return big;
-    const int least = r.per_cu <= 8 ? 2 : r.per_cu <= 12 ? (r.units >= 5 ? 16 : 3) : (r.units >= 5 ? 8 : 16);
+    int least = r.units >= 8 || r.per_cu <= 6 ? 1 : r.per_cu <= 8 || r.words >= 4 ? 2 : 3;
+    if (tsa_rounds(r.per_cu, 28 / big, r.lds) > rounds_one) {
+      if (big == 2) return 1;
+      if (r.units >= 8) least = rounds_one == 1 || r.per_cu > 12 ? 2 : 1;
+      else least = r.per_cu <= 8 || rounds_one > 1 ? 8 : 16;
+    }
     return nsweeps < least ? 1 : big;
   }
-  // The loop's chains stay from its first level to its last: one wave keeps twelve of them resident on a unit, two
-  // waves eight (sat30, 3072 chains, ten levels of ten sweeps: 1324 against 1660 us), four waves four (sat100: 2646
-  // against 3656).
-  if (kind == TSA_TEAM_LOOP && !r.moves && r.units < 8) {
-    if (r.per_cu > (r.units >= 5 ? 6 : 8)) return 1;
-    if (r.nint < 64 && nsweeps < 2) return 1;
+  // The loop's chains stay from its first level to its last, so all of them want to be resident at once: 16 waves of
+  // k_team's loop a unit, 12 of k_sweep's (3072 chains of sat30, ten levels of ten sweeps: one wave 1324 us, two 1660;
+  // 2048 chains of sat70, ten of five: 999 and 1296, 1792 chains 985 and 869).  With one sweep a level the loop's time is
+  // the levels' folds, which a team makes beside the next sweep: a second round of it is worth it where the sweep is
+  // short or wide (sq12, 2048 chains: one wave 635, four 560; sat30, 3072 chains: 674 and 626), unless the tree is
+  // less than one scan of a wave.
+  if (kind == TSA_TEAM_LOOP && !r.moves) {
+    if (nsweeps < 2 && r.nint < 64) return 1;
+    if (tsa_rounds(r.per_cu, 8, r.lds_loop) == 1) return 2;
+    if (nsweeps < 2 && (r.words >= 4 || r.units < 4)) return big;
+    if (tsa_rounds(r.per_cu, 12, r.lds_one) == 1 && !(r.units >= 8 && r.per_cu <= 6)) return 1;
   }
   return big;
 }
