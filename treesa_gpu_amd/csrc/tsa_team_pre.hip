@@ -119,6 +119,28 @@ __global__ void __launch_bounds__(64 * (1 + TSA_DRAW_HELPERS))
       if (MODE != 0) cfold.z[i] = cc.z[i];
     }
   };
+  // The level's entry of the schedule, and the next one's, read a level ahead: at a level's end every wave goes by it at
+  // once, where a read would be two round trips to memory on the sweeping wave's path (256 chains of sat100, 100 levels of
+  // one sweep, 2147 -> 2081 us).
+  int ev = 0, ev_next = 0, left_next = 0;
+  float beta_next = beta;
+  auto read_ahead = [&]() {
+    const int k = lv + 1 < Lv.nlev ? lv + 1 : lv;
+    ev_next = Lv.eval[k];
+    left_next = Lv.niters[k];
+    beta_next = Lv.beta[k];
+  };
+  auto next_level = [&]() {
+    lv++;
+    ev = ev_next;
+    left = left_next;
+    beta = beta_next;
+    read_ahead();
+  };
+  if constexpr (LVL) {
+    ev = Lv.eval[0];
+    read_ahead();
+  }
   int np = 0, na = 0, nst = 0, nv = 0;
   // The sweeping wave and the helpers run loops of their own, which meet at the same workgroup barriers: one per sweep,
   // one more at an evaluated level's end.
@@ -131,7 +153,6 @@ __global__ void __launch_bounds__(64 * (1 + TSA_DRAW_HELPERS))
       __syncthreads();
       if constexpr (LVL) {
         if (--left == 0) {  // the level's last sweep
-          const int ev = F->Lv.eval[lv];
           if (ev >= 0) {
             keep_costs();
             const int slot = own.slot < 0 ? 0 : own.slot ^ 1;
@@ -139,7 +160,7 @@ __global__ void __launch_bounds__(64 * (1 + TSA_DRAW_HELPERS))
             __syncthreads();
             if (wv == 1) own = tsa_team_fold_end<W, MODE>(F, 0, -INFINITY, ev, lv, own, slot);
           }
-          if (++lv < F->Lv.nlev) left = F->Lv.niters[lv];
+          next_level();
         }
       }
     }
@@ -205,14 +226,11 @@ __global__ void __launch_bounds__(64 * (1 + TSA_DRAW_HELPERS))
       __syncthreads();
       if constexpr (LVL) {
         if (--left == 0) {
-          if (F->Lv.eval[lv] >= 0) {
+          if (ev >= 0) {
             keep_costs();
             __syncthreads();
           }
-          if (++lv < F->Lv.nlev) {
-            beta = F->Lv.beta[lv];
-            left = F->Lv.niters[lv];
-          }
+          next_level();
         }
       }
     }
