@@ -294,27 +294,21 @@ __global__ void __launch_bounds__(SUMS || SLICE ? 512 : 1024) k_wide(TsaKParams 
       // 1. scan: a wave takes 64-node groups; each lane reads its node's priority, parent and children
       // words, then the three neighbour priorities, in two rounds of independent LDS reads (tsa_scan_active:
       // no branches, so that every read of a round is in flight at once)
-      // a wave takes its groups up to eight at a time: their ballots, then (one workgroup per chain) one append; a
-      // batch reads as many as it has, rounded up to a power of two (eight whatever there were: 300 chains of a
-      // 3-regular graph n=600, ten groups for eight waves, eight sweeps 360 us, now 279)
-      auto scan = [&](auto batch, int g0) {
-        constexpr int Q = decltype(batch)::value;
-        uint64_t bb[Q];
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-          const int gi = g0 + q * nwv;
-          const int i = gi * 64 + lane;
-          const int ic = i < nint ? i : nint - 1;
-          const uint32_t pv = pri[ic], p = par[ic], cw = ch[ic];
-          const uint32_t kp = tsa_pri_key(pri, (uint32_t)m - 1u, p), kl = tsa_pri_key(pri, (uint32_t)m - 1u, cw & 0xFFFFu),
-                         kr = tsa_pri_key(pri, (uint32_t)m - 1u, cw >> 16);
-          const bool act = tsa_scan_active((uint32_t)(m + ic), pv, kp, kl, kr) & (gi < ngrp) & (i < nint);
-          bb[q] = __ballot(act);
-          if (COOP && lane == 0 && gi < ngrp) masks[gi] = bb[q];
-        }
+      auto group = [&](int gi) {
+        const int i = gi * 64 + lane;
+        const int ic = i < nint ? i : nint - 1;
+        const uint32_t pv = pri[ic], p = par[ic], cw = ch[ic];
+        const uint32_t kp = tsa_pri_key(pri, (uint32_t)m - 1u, p), kl = tsa_pri_key(pri, (uint32_t)m - 1u, cw & 0xFFFFu),
+                       kr = tsa_pri_key(pri, (uint32_t)m - 1u, cw >> 16);
+        const uint64_t b = __ballot(tsa_scan_active((uint32_t)(m + ic), pv, kp, kl, kr) & (gi < ngrp) & (i < nint));
+        if (COOP && lane == 0 && gi < ngrp) masks[gi] = b;
+        return b;
+      };
+      // one workgroup per chain: the active nodes of a batch are appended (any order will do: the visits of a phase
+      // commute and every entry carries its own node id)
+      auto append = [&](const auto& bb, int g0) {
         if constexpr (!COOP) {
-          // one workgroup per chain: append the active nodes (any order will do: the visits of a phase
-          // commute and every entry carries its own node id)
+          constexpr int Q = sizeof(bb) / sizeof(bb[0]);
           int tot = 0;
 #pragma unroll
           for (int q = 0; q < Q; q++) tot += __popcll(bb[q]);
@@ -329,14 +323,28 @@ __global__ void __launch_bounds__(SUMS || SLICE ? 512 : 1024) k_wide(TsaKParams 
           }
         }
       };
+      // a wave takes its groups up to eight at a time, every read of the batch in flight at once
       if constexpr (SUMS) {  // (trees with sets this wide have groups for a full batch)
-        for (int g0 = wv; g0 < ngrp; g0 += 8 * nwv) scan(TsaLaneStep<8>{}, g0);
+        for (int g0 = wv; g0 < ngrp; g0 += 8 * nwv) {
+          uint64_t bb[8];
+#pragma unroll
+          for (int q = 0; q < 8; q++) bb[q] = group(g0 + q * nwv);
+          append(bb, g0);
+        }
       } else {
+        // a batch reads as many as it has, rounded up to a power of two (eight whatever there were: 300 chains of a
+        // 3-regular graph n=600, ten groups for eight waves, eight sweeps 360 us, now 279)
+        auto batch = [&](auto n, int g0) {
+          uint64_t bb[decltype(n)::value];
+#pragma unroll
+          for (int q = 0; q < decltype(n)::value; q++) bb[q] = group(g0 + q * nwv);
+          append(bb, g0);
+        };
         for (int g0 = __builtin_amdgcn_readfirstlane(wv); g0 < ngrp; g0 += 8 * nwv) {
-          if (g0 + 4 * nwv < ngrp) scan(TsaLaneStep<8>{}, g0);
-          else if (g0 + 2 * nwv < ngrp) scan(TsaLaneStep<4>{}, g0);
-          else if (g0 + nwv < ngrp) scan(TsaLaneStep<2>{}, g0);
-          else scan(TsaLaneStep<1>{}, g0);
+          if (g0 + 4 * nwv < ngrp) batch(TsaLaneStep<8>{}, g0);
+          else if (g0 + 2 * nwv < ngrp) batch(TsaLaneStep<4>{}, g0);
+          else if (g0 + nwv < ngrp) batch(TsaLaneStep<2>{}, g0);
+          else batch(TsaLaneStep<1>{}, g0);
         }
       }
       __syncthreads();
