@@ -68,3 +68,31 @@ def test_team_pre_wide_frontiers(mode):
 
 def test_team_pre_many_chains_one_sweep_per_level():
     compare(network("sat", 30), "tc", 300, True, niters=1)
+
+
+# tc mode, one lane per proposal: few sweeps a launch or level run k_team_pre, many the one-wave kernel's helper form
+@pytest.mark.parametrize("kind,size", [("sat", 30), ("sat", 100)])
+@pytest.mark.parametrize("niters", [3, 9])
+def test_either_kernel_by_the_sweeps(kind, size, niters):
+    for chains in (9, 200):
+        for anneal in (False, True):
+            compare(network(kind, size), "tc", chains, anneal, niters=niters)
+
+
+def test_both_kernels_in_one_session():
+    inst, outs = network("sat", 30), []
+    lay = capi.layout(inst.m, inst.nlab)
+    for draw in (1, -1):
+        cfg = capi.make_config(mode="tc", sc_target=8.0, seed=5, fused_energy=True, draw_waves=draw, level_loop=1)
+        trees = np.stack([host.random_tree(inst.m, 11 + k) for k in range(4)])
+        with capi.Context(lay, inst.leaf(lay.W), inst.leaf_sc, cfg, 40) as ctx:
+            ctx.upload(inst.population(lay, trees, 40, seed=5))
+            ctx.track_begin("tc", sc_target=8.0, max_levels=9)
+            for k, n in enumerate((1, 7, 2)):
+                ctx.anneal(capi.ORDER_PREORDER, [0.5 + 3 * k, 1.0 + 3 * k, 2.0 + 3 * k], [n] * 3, [1, 1, 1],
+                           sweep0=30 * k, level0=3 * k)
+            chain, level, score, rec, rows, _, _ = ctx.track_end()
+            outs.append([np.array([chain, level]), np.array(score), rec, rows["lc"], rows["chain"], rows["meanE"],
+                         ctx.download(), np.array(ctx.stats())])
+    for a, b in zip(*outs):
+        np.testing.assert_array_equal(a, b)

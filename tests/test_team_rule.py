@@ -85,3 +85,19 @@ def test_blocks_of_levels(waves, chains, tree, want):
 
 def test_asked(waves):
     assert [waves("sat30", 8192, 1, asked=a) for a in (2, 3, 8)] == [2, 3, 8]
+
+
+def test_preorder_of_narrow_sets_keeps_one_wave_for_many_sweeps(tmp_path):
+    """k_team_pre or k_sweep's helper form (tsa_pre_pays), where one was measured ahead by more than the runs differ."""
+    exe = str(tmp_path / "pre")
+    subprocess.run(["g++", "-O1", "-I", os.path.join(HERE, "..", "treesa_gpu_amd", "csrc"),
+                    os.path.join(HERE, "pre_rule_check.cpp"), "-o", exe], check=True)
+    # mode, words, fewer chains than half the compute units, kind, sweeps (of the launch or a level)
+    one = [(0, 1, 1, SWEEPS, 8), (0, 1, 1, SWEEPS, 50), (0, 1, 0, SWEEPS, 50), (0, 2, 1, SWEEPS, 16), (0, 2, 0, SWEEPS, 50),
+           (0, 1, 1, LOOP, 5), (0, 1, 1, LOOP, 50)]
+    team = [(0, 1, 1, SWEEPS, 2), (0, 1, 0, SWEEPS, 4), (0, 2, 1, SWEEPS, 4), (0, 2, 0, SWEEPS, 8), (0, 1, 1, LOOP, 1),
+            (0, 1, 0, LOOP, 50), (0, 2, 1, LOOP, 25), (0, 4, 1, SWEEPS, 50), (0, 8, 1, LOOP, 50), (1, 1, 1, SWEEPS, 50),
+            (2, 2, 1, LOOP, 50)]
+    text = "\n".join(" ".join(map(str, c)) for c in one + team)
+    got = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert got == ["0"] * len(one) + ["1"] * len(team)

@@ -77,7 +77,8 @@ struct TsaLaunch {
   int team_fits;
   TsaTeamRule team_rule;
   int team_full, team;
-  int team_pre;      // pre-order sweeps with helper waves (draw_waves) run k_team_pre
+  int team_pre;      // pre-order sweeps with helper waves (draw_waves) can run k_team_pre
+  int pre_sparse;    // fewer chains than half the compute units (tsa_pre_pays)
 };
 
 // Helper waves per workgroup of a pre-order sweep with draws made ahead (the workgroup fills a compute unit's
@@ -191,7 +192,7 @@ hipError_t tsa_launch_sweeps_sliced(const TsaLaunch& L, int mode, int order, con
                                     hipEvent_t e0, hipEvent_t e1, const TsaLevels* lv, int* res);
 // Waves per chain of a par launch of the LDS kernels (1: k_sweep); nsweeps as tsa_team_waves takes it.
 int tsa_par_waves(const TsaLaunch& L, int mode, const TsaKParams& P, TsaTeamKind kind, int nsweeps);
-// Whether pre-order sweeps run k_team_pre.
+// Whether pre-order sweeps can run k_team_pre (tsa_pre_pays: whether a launch of them does).
 bool tsa_pre_team(const TsaLaunch& L, int mode, const TsaKParams& P);
 // Par sweeps with L.team waves per chain (tsa_team.h): work-list entries long (L.team_full) or short, without and with
 // slicing; res as above.

@@ -283,7 +283,9 @@ hipError_t tsa_launch_sweeps(const TsaLaunch& L, int mode, int order, const TsaK
                               : (L.team_full ? tsa_launch_team_full : tsa_launch_team_compact);
     return go(T, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
   }
-  if (order == 1 && tsa_pre_team(L, mode, P))
+  if (order == 1 && tsa_pre_team(L, mode, P) &&
+      tsa_pre_pays(mode, P.W, L.pre_sparse != 0, lv ? TSA_TEAM_LOOP : TSA_TEAM_SWEEPS,
+                   lv ? (lv->nlev > 0 ? lv->total / lv->nlev : 0) : nsweeps))
     return tsa_launch_team_pre(L.W, mode, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st, e0, e1, lv, res);
   if (P.slicing)
     return tsa_launch_sweeps_sliced(L, mode, order, P, rec, leaf, fix, nchains, beta, sweep0, nsweeps, stats, eo, st,

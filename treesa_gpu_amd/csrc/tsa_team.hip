@@ -13,6 +13,7 @@ void tsa_team_plan(const TsaKParams& P, int nchains, int ncu, int lds_max, int w
   L->team_fits = L->team_full = 0;
   if (want > 8) want = 0;  // (a plan for the wide kernel: it says nothing here)
   L->team_pre = want != 1 && tsa_team_pre_fits(P, lds_max);
+  L->pre_sparse = 2ll * nchains < ncu;
   if (want == 1 || P.par_follow || P.par_band > 0) return;
   // the most LDS any launch of the context asks for: a float mode's cache, the level loop, slice moves
   const bool moves = P.slicing && P.slice_moves > 0;

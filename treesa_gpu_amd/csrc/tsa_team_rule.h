@@ -1,5 +1,5 @@
-// tsa_team_rule.h -- how many waves sweep a chain in par order (k_team, or 1: k_sweep).  Plain C++, also compiled by the
-// CPU tests.
+// tsa_team_rule.h -- how many waves sweep a chain in par order (k_team, or 1: k_sweep), and which kernel sweeps in pre-order
+// with helper waves (k_team_pre, or k_sweep's helper form).  Plain C++, also compiled by the CPU tests.
 #pragma once
 
 // What the choice goes by.
@@ -96,4 +96,22 @@ static inline int tsa_team_waves_float(const TsaTeamRule& r, int mode, TsaTeamKi
 static inline int tsa_team_waves(const TsaTeamRule& r, int mode, TsaTeamKind kind, int nsweeps) {
   if (r.asked > 0) return r.asked;
   return mode == 0 ? tsa_team_waves_tc(r, kind, nsweeps) : tsa_team_waves_float(r, mode, kind, nsweeps);
+}
+
+// Whether pre-order sweeps with helper waves run k_team_pre.  In tc mode and with a proposal on one lane its steps are no
+// shorter than k_sweep's (a visit saves P's set and two look-ups and pushes entries of four words), only its start and its
+// levels' ends, so that k_sweep is ahead from some sweeps on, the sooner the fewer chains there are.  k_sweep's time over
+// k_team_pre's, launch of sweeps and energies / levels of the loop:
+//                        4 sweeps    8     16     50     20 levels of 1    2     5     8 levels of 25
+//   sat40,  16 chains      0.98    0.96   0.94   0.93          1.00      0.98  0.98       0.99
+//           64             1.01    0.99   0.96   0.96          1.01      1.00  0.99       1.00
+//          256             1.02    1.00   1.00   0.99          1.02      1.03  1.02       1.02
+//   sat100, 16 (2 words)   1.01    1.00   0.98   0.97          1.00      1.00  0.99       1.01
+//          256             1.02    1.01   1.00   0.99          1.07      1.04  1.03       1.02
+// (43 chains of sat22, 65 levels of 50 sweeps: 32.3 ms with k_team_pre, 30.9 with k_sweep; 200 chains, 30 levels: 13.3,
+// 13.5.)  W: 64-bit words per label set; sparse: fewer chains than half the compute units; nsweeps as above.
+static inline bool tsa_pre_pays(int mode, int W, bool sparse, TsaTeamKind kind, int nsweeps) {
+  if (mode != 0 || W > 2) return true;
+  if (kind == TSA_TEAM_LOOP) return W > 1 || !sparse || nsweeps <= 2;
+  return nsweeps <= (W > 1 || !sparse ? 8 : 4);
 }
