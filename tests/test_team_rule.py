@@ -101,3 +101,27 @@ def test_preorder_of_narrow_sets_keeps_one_wave_for_many_sweeps(tmp_path):
     text = "\n".join(" ".join(map(str, c)) for c in one + team)
     got = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split()
     assert got == ["0"] * len(one) + ["1"] * len(team)
+
+
+def test_slice_moves_keep_chains_resident(tmp_path):
+    """Ten sweeps with slice moves: two waves while they take no more rounds of resident chains than one wave each does."""
+    exe = str(tmp_path / "rule")
+    subprocess.run(["g++", "-O1", "-I", os.path.join(HERE, "..", "treesa_gpu_amd", "csrc"),
+                    os.path.join(HERE, "team_rule_check.cpp"), "-o", exe], check=True)
+
+    def waves(nint, W, per_cu, nsweeps):
+        n4, leaf, rec = (nint + 3) // 4 * 4, (nint + 1) * W * 8, nint * (W * 8 + 4) + W * 8
+        lds = 163840 // (leaf + rec + n4 * 22 + 16 + 2640)  # short entries, two caches
+        lanes = max(1, W // 2)
+        line = [0, per_cu, nint * lanes // 64, nint * max(2, lanes) // 64, nint, 1, lds, 0, resident(nint, W, per_cu)[2], W, 0,
+                SWEEPS, nsweeps]
+        return int(subprocess.run([exe], input=" ".join(map(str, line)), capture_output=True, text=True, check=True).stdout)
+
+    sat40, sat60, sat70, sat85, sat100, sq10, sq12 = (170, 1), (255, 1), (297, 2), (361, 2), (425, 2), (99, 4), (143, 8)
+    for tree, per_cu in ((sat40, 10), (sat60, 10), (sat70, 8), (sat85, 6), (sat100, 5), (sq10, 8), (sq12, 16)):
+        assert waves(*tree, per_cu, 1) == waves(*tree, per_cu, 10) == 2, (tree, per_cu)
+    for tree, per_cu in ((sat40, 12), (sat70, 12), (sat85, 8), (sat100, 8), (sat100, 12)):
+        assert waves(*tree, per_cu, 1) == waves(*tree, per_cu, 10) == 1, (tree, per_cu)
+    for tree, per_cu in ((sat60, 12), (sq10, 10)):
+        assert waves(*tree, per_cu, 1) == 1 and waves(*tree, per_cu, 10) == 2, (tree, per_cu)
+    assert waves(*sq10, 16, 1) == 2

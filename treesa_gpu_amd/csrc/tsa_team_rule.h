@@ -24,6 +24,27 @@ static inline int tsa_rounds(int per_cu, int waves, int lds) {
   return (per_cu + most - 1) / (most > 0 ? most : 1);
 }
 
+// Sweeps with slice moves of five chains per unit and more (tc mode): two waves, or one where they take more rounds of
+// resident chains.  The registers let 20 waves of k_team with slice moves share a unit with one word per label set and 16
+// with more, of k_sweep 16 with one or two words, 12 with four, 4 with eight.  Ten sweeps and the energies, us, one wave /
+// two, by chains per unit (*: a round more of teams):
+//              6           7            8            10           12           16
+//   sat40   271 / 199   270 / 200    272 / 204    311 / 232    317 / 332*   367 / 386*
+//   sat60   324 / 227   327 / 228    328 / 235    379 / 265    385 / 370*   451 / 435*
+//   sat70   386 / 275   388 / 276    389 / 282    452 / 444*   456 / 469*   534 / 592*
+//   sat85   426 / 305   430 / 450*   432 / 483*   504 / 513*   510 / 570*   765 / 755*
+//   sat100  468 / 493*  470 / 537*   473 / 554*   557 / 609*   563 / 774*   838 / 968*
+//   sq10    263 / 189   265 / 190    267 / 197    315 / 298*   317 / 316*   466 / 381
+// and of one sweep (12 chains per unit) sat60 64 / 70*, sat100 87 / 115*, sq10 59 / 69*.  With one word of several
+// wavefuls and with four words a round more still pays from a few sweeps on.
+static inline int tsa_team_moves_tc(const TsaTeamRule& r, int nsweeps) {
+  if (r.nint < 64 && nsweeps < 2) return 1;
+  const int team = r.words <= 1 ? 20 : 16, one = r.words <= 2 ? 16 : r.words <= 4 ? 12 : 4;
+  if (tsa_rounds(r.per_cu, team / 2, r.lds) <= tsa_rounds(r.per_cu, one, r.lds_one)) return 2;
+  if (r.words >= 4) return nsweeps < 2 ? 1 : 2;
+  return r.words <= 1 && r.units >= 3 && nsweeps >= 4 ? 2 : 1;
+}
+
 // The lines lie where the measured times cross (par order, blocks of levels, 40 levels of one sweep, us):
 //   chains  sat100: one wave / team of 2 / 4 / 8    sat60                     sq14 (8 words)
 //      72            917 / 698 / 548 / 530          692 / 492 / 468 / 475      917 / 632 / 534 / 507
@@ -33,7 +54,7 @@ static inline int tsa_rounds(int per_cu, int waves, int lds) {
 //    6144           3372 / 3908 / 3546 / 5093      1894 / 1891 / 2319 / 3620
 // Eight waves pay while a compute unit has one chain; beyond that four where a tree's nodes (times the lanes of a
 // proposal) fill them, else two; from 16 chains per unit on, one wave each hides its latency behind the others'.  With
-// slice moves a chain holds a second cost cache, and from five chains per unit on two waves keep all of them resident
+// slice moves a chain holds a second cost cache, and from five chains per unit on two waves keep more of them resident
 // (sat70, 2048 chains: 6.9 ms against 10.2 with four).
 static inline int tsa_team_waves_tc(const TsaTeamRule& r, TsaTeamKind kind, int nsweeps) {
   if (r.per_cu > 16) return 1;
@@ -56,7 +77,7 @@ static inline int tsa_team_waves_tc(const TsaTeamRule& r, TsaTeamKind kind, int 
   const int waves_one = r.words <= 2 ? 24 : r.words <= 4 ? 20 : 16;
   const int rounds_one = tsa_rounds(r.per_cu, waves_one, r.lds_one);
   if (kind == TSA_TEAM_SWEEPS) {
-    if (r.moves) return r.nint < 64 && nsweeps < 2 ? 1 : big;
+    if (r.moves) return tsa_team_moves_tc(r, nsweeps);
     int least = r.units >= 8 || r.per_cu <= 6 ? 1 : r.per_cu <= 8 || r.words >= 4 ? 2 : 3;
     if (tsa_rounds(r.per_cu, 28 / big, r.lds) > rounds_one) {
       if (big == 2) return 1;
