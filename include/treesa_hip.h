@@ -76,13 +76,15 @@ typedef struct tsa_config_t {
   float v2_l3launch, v2_lperm2, v2_lcc_bit, v2_lcc_cell, v2_ltc_bit, v2_ltc_pad, v2_ltc_out, v2_lsmall_cell;
   int32_t v2_small_rank;
   /* wide kernel plan (0 = automatic): waves per workgroup (1..16), workgroups per chain (1..16).  On contexts whose
-   * chains sit in LDS, wide_waves is the waves per chain of par sweeps (1: one, 2..8; 0 automatic) */
+   * chains sit in LDS, wide_waves is the waves per chain of par sweeps (1: one, 2..8; 0 and 9..16 automatic: by the
+   * chains per compute unit, the tree, the mode and the sweeps of the launch); the binary's --wpc plans the wide
+   * kernel only */
   int32_t wide_waves, wide_wgs;
   /* 1: every tsa_sweeps on the register-width path also leaves the energies of the swept population ready,
    * so that tsa_energy / tsa_track launch no energy kernel; for callers that evaluate after every level.  The
-   * sweep kernel computes every node's cost while the chain is still staged in LDS and folds it there, or,
-   * with more than twice the chains that fit on the device at once (or with 2), leaves the costs to a fold
-   * kernel that folds every chain in one round.  The wide path keeps a node-cost cache instead and its energy call
+   * sweep kernel has every node's cost while the chain is still staged in LDS and folds them there, or,
+   * with more than twice the chains that fit on the device at once (or with 2, or in a block of levels), leaves the
+   * costs to a fold kernel that folds every chain in one round.  The wide path keeps a node-cost cache instead and its energy call
    * only folds it. */
   int32_t fused_energy;
   /* chunk summaries of the wide kernel (the reference's --sums / --no-sum, csrc/treesa_gpu.cu:1444-1448):
@@ -97,21 +99,26 @@ typedef struct tsa_config_t {
   int32_t track_overlap;
   /* pre-order sweeps: one chain per workgroup, whose three helper waves draw every internal node's random
    * numbers (the rule word and the Metropolis threshold) for the next sweep while the first wave sweeps, instead
-   * of each visit drawing its own: 0 = automatic (on for at most one chain per compute unit, where the sweeping
-   * wave's dependent steps bound the sweep and three SIMDs idle), 1 = on, -1 = off.  Results do not change */
+   * of each visit drawing its own: 0 = automatic (on for at most one chain per compute unit), 1 = on, -1 = off.  Without
+   * slicing the sweeping wave then also keeps a cost cache and passes a node's words on with its work-list entry (in tc
+   * mode with sets of one or two words only for launches or levels of few sweeps), which is faster up to four chains
+   * per compute unit (tc mode; the float modes at least up to eight).  Results do not change */
   int32_t draw_waves;
   /* wide kernel with several workgroups per chain: polls a workgroup waits at the chain's check-in for the
    * others before it sweeps the chain alone (0 = default, about a millisecond; -1 = at once, every chain swept
    * by one workgroup -- for tests).  Results do not change */
   int32_t wide_join;
-  /* tsa_anneal: 0 = automatic (the level loop in one launch when every chain of it is resident on the device
-   * at once, else one sweep launch and one selection per level), 1 = the level loop in one launch whenever the
-   * context's kernels run it, -1 = per-level launches.  Results do not change */
+  /* tsa_anneal, on contexts whose chains sit in LDS: 0 = automatic (blocks of levels in par order with fused_energy,
+   * without slicing and with the overlapped selection; else the level loop in one launch when every chain of it is
+   * resident on the device at once; else one sweep launch and one selection per level), 1 = the level loop in one
+   * launch, -1 = no level loop (launches per level, or blocks with more than twice the chains the device holds at
+   * once).  Results do not change */
   int32_t level_loop;
-  /* tsa_anneal without the one-launch level loop, on the one-wave LDS kernels whose selection overlaps the next
-   * sweep with the fold apart (more than twice the chains the device holds at once, par order, no slicing):
-   * levels per sweep launch, each evaluated level leaving its own snapshot for the fold and the selection
-   * (0 = automatic: 8, the most; 1 = one level per launch).  Results do not change */
+  /* tsa_anneal in blocks of levels (level_loop; and the wide path with chunk summaries, tc mode, par order and fewer
+   * chains than compute units): levels per sweep launch, each evaluated level leaving its own snapshot for the fold
+   * and the selection beside the next block's sweeps (0 = automatic: 8, the most; 1 = no blocks).  The snapshots take
+   * about 10 bytes per node and chain for each of 3 * level_blocks levels, or of the session's if those are fewer;
+   * where they cannot be allocated, the call runs the level loop or launches per level.  Results do not change */
   int32_t level_blocks;
 } tsa_config_t;
 
@@ -230,14 +237,19 @@ int tsa_track_end(tsa_ctx* ctx, int32_t* best_chain, int32_t* best_level, double
  * tsa_track at the evaluated ones: the same population, statistics, trace rows and, at tsa_track_end, the
  * same best chain, level, score and tree.  It replaces the level loop of run_anneal
  * (csrc/treesa_gpu.cu:1788-1832), which the reference runs as one sweep launch and one host-side selection per
- * level.  On the LDS kernels with every chain resident at once (tsa_config_t.level_loop) the call is ONE
- * launch: each chain stays staged from its first level to its last, folds its energy and keeps its own best
- * tree after every evaluated level, and the last chain to finish a level selects while the others sweep on, so
- * no level waits for the host or for a launch (the trace row's ticks: the device clock of that selection).
- * Else it runs those per-level launches itself.  Needs tsa_track_begin (max_levels >= level0 + nlevels); a
- * session that has called tsa_track runs per-level launches, and tsa_track after a one-launch tsa_anneal in the
- * same session fails.  tsa_describe names the way the last call ran.  The kernel time counts in
- * tsa_sweeps_ms.  Asynchronous. */
+ * level.  It runs one of three ways (tsa_config_t.level_loop, level_blocks; tsa_describe names the last call's):
+ *   - blocks of levels (par order without slicing, with fused_energy): one sweep launch per block, its levels' folds and
+ *     selections on a second stream beside the next block's sweeps; a call of a single level is a launch of its own;
+ *   - the level loop (the LDS kernels with every chain resident at once): ONE launch.  Each chain stays staged from its
+ *     first level to its last, folds its energy and keeps its own best tree after every evaluated level, and the last
+ *     chain to finish a level selects while the others sweep on (the trace row's ticks: the device clock of that
+ *     selection);
+ *   - launches per level.
+ * Asynchronous: where every chain is resident at once no level waits for the host.  With more chains, and on the wide
+ * path, the call may wait on the host for the selection of a level (or block) three back before it enqueues the next.
+ * Needs tsa_track_begin (max_levels >= level0 + nlevels).  Calls of one session may differ in order.  A session that has
+ * called tsa_track runs no level loop, and tsa_track fails in a session whose levels tsa_anneal ran by the level loop or
+ * could have (every chain resident, level_loop not -1).  The kernel time counts in tsa_sweeps_ms. */
 int tsa_anneal(tsa_ctx* ctx, int32_t order, int32_t level0, int32_t nlevels, const float* betas,
                const int32_t* niters, const uint8_t* evaluated, uint32_t sweep0);
 

@@ -458,7 +458,9 @@ static int plan_one_wave(const tsa_layout_t* lay, const tsa_config_t* cfg, int n
   }
   L->lds_max = ldsw * 8;
   // pre-order sweeps of at most one chain per compute unit are bound by the sweeping wave's chain of
-  // dependent steps while three SIMDs idle: there helper waves draw the next sweep's random numbers
+  // dependent steps while three SIMDs idle: there helper waves draw the next sweep's random numbers.  (The line is
+  // k_sweep's helper form's.  k_team_pre, which runs without slicing, is ahead further: four sweeps, us, without / with
+  // helpers, sat100: tc mode 512 chains 123 / 109, 1024 122 / 109, 2048 147 / 187; gpu mode 1024 501 / 207, 2048 555 / 398.)
   L->draw_waves = cfg->draw_waves > 0 || (cfg->draw_waves == 0 && ncu > 0 && (long long)nchains <= ncu);
   *use_lds_out = use_lds;
   return TSA_OK;

@@ -120,7 +120,7 @@ const std::vector<Flag>& flags() {
       {"--wide", nullptr, "runtime-width label sets whatever the label count", SWITCH(wide, true)},
       {"--sums", nullptr, "chunk summaries on", SWITCH(force_sum, true)},
       {"--no-sum", nullptr, "chunk summaries off", SWITCH(no_sum, true)},
-      {"--wpc", "n", "wide kernel: 32-lane warps per workgroup (waves = n / 2)", INT_FIELD(wpc)},
+      {"--wpc", "n", "wide kernel: 32-lane warps per workgroup (waves = n / 2); no effect in LDS", INT_FIELD(wpc)},
       {"--wide-wgs", "K", "wide kernel: workgroups per chain", INT_FIELD(wide_wgs)},
       {"--wide-lanes", "G", "wide kernel: lanes per proposal", INT_FIELD(wide_lanes)},
       {"--draw-waves", "1|-1|0",
@@ -152,12 +152,12 @@ const std::vector<Flag>& flags() {
       {"--host-select", nullptr, "select on the host at every level, also for --scheme indep",
        SWITCH(host_select, true)},
       {"--no-overlap", nullptr, "device-side selection on the sweep's stream", SWITCH(no_overlap, true)},
-      {"--level-launches", nullptr, "scheme indep: one sweep launch and one selection per level, not the level loop "
-       "in one launch", SWITCH(level_launches, true)},
+      {"--level-launches", nullptr, "scheme indep: one sweep launch and one selection per level, not blocks of levels or "
+       "the level loop", SWITCH(level_launches, true)},
       {"--level-loop", nullptr, "scheme indep: the level loop in one launch also with more chains than are resident "
        "at once", SWITCH(level_loop, true)},
-      {"--level-blocks", "K", "scheme indep, par order, more than twice the chains the device holds at once: levels "
-       "per sweep launch (0: automatic, 1: one)", INT_FIELD(level_blocks)},
+      {"--level-blocks", "K", "scheme indep, par order without slicing: levels per sweep launch (0: automatic, 8; 1: no "
+       "blocks)", INT_FIELD(level_blocks)},
       {"--level-log", "FILE", "one JSON line per evaluated level: best chain, score, energies, ancestors",
        TEXT_FIELD(level_log)},
   };
